@@ -322,6 +322,24 @@ int awq_silu_mul(const void* gate_up, void* out, int64_t M, int64_t I, void* str
 int awq_fp16_linear(const void* x, const void* weight, void* out, int64_t M, int64_t N, int64_t K,
                     void* stream);
 
+/* Attention of one new position over a static KV cache (the decode step of
+ * model/qwen2.py:104-163): rotate-half RoPE of q and k (fp32), k (rounded to
+ * fp16) and v stored at row *pos of the caches, softmax(q K^T / sqrt(head_dim))
+ * V over positions 0 .. *pos in fp32, out fp16.  qkv fp16 [(num_heads + 2
+ * num_kv_heads) * head_dim]; k_cache / v_cache fp16 [num_kv_heads, max_seq,
+ * head_dim]; cos / sin fp32 [max_seq, head_dim]; pos int64 [1] on the device
+ * (outside 0 .. max_seq - 1 nothing is written); out fp16 [num_heads *
+ * head_dim].  head_dim 64 or 128 (AWQ_ERR_PATH otherwise), num_heads a
+ * multiple of num_kv_heads.  workspace: at least
+ * awq_fp16_attention_decode_workspace bytes, of any content; it holds nothing
+ * between calls.  Two launches. */
+size_t awq_fp16_attention_decode_workspace(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                           int64_t max_seq);
+int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                              const int64_t* pos, void* out, int64_t num_heads, int64_t num_kv_heads,
+                              int64_t head_dim, int64_t max_seq, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 #ifdef __cplusplus
 }
 #endif

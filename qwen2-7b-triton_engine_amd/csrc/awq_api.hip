@@ -58,6 +58,15 @@ int check_dims(int64_t M, int64_t N, int64_t K, int32_t G) {
     return AWQ_OK;
 }
 
+// Shapes of the attention entry points: heads of 64 or 128 columns, head
+// counts that fit a grid's y and z, one layer's cache below 2^31 bytes.
+int check_attention(int64_t nh, int64_t kvh, int64_t hd, int64_t max_seq) {
+    if (nh <= 0 || kvh <= 0 || nh % kvh != 0 || max_seq <= 0) return AWQ_ERR_BAD_DIMS;
+    if (hd != 64 && hd != 128) return AWQ_ERR_PATH;
+    if (nh > 4096 || max_seq > kIndexLimit || kvh * max_seq > kBytesLimit / (2 * hd)) return AWQ_ERR_TOO_LARGE;
+    return AWQ_OK;
+}
+
 // Workspace bytes of a plan that keeps fp32 partials [split, M, N].
 uint64_t partials_workspace(int64_t split, int64_t M, int64_t N) {
     return kPartialsOffset + (uint64_t)split * (uint64_t)M * (uint64_t)N * 4u;
@@ -1160,6 +1169,40 @@ int awq_fp16_linear(const void* x, const void* weight, void* out, int64_t M, int
     const hipError_t e = launch_fp16_gemv(static_cast<const half_t*>(x), static_cast<const half_t*>(weight),
                                           static_cast<half_t*>(out), (int)M, (int)N, (int)K, (int)cus(),
                                           static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
+}
+
+size_t awq_fp16_attention_decode_workspace(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                           int64_t max_seq) {
+    if (check_attention(num_heads, num_kv_heads, head_dim, max_seq) != AWQ_OK) return 0;
+    return decode_attn_workspace((int)max_seq, (int)num_heads, (int)head_dim);
+}
+
+int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                              const int64_t* pos, void* out, int64_t num_heads, int64_t num_kv_heads,
+                              int64_t head_dim, int64_t max_seq, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+    const int st = check_attention(num_heads, num_kv_heads, head_dim, max_seq);
+    if (st != AWQ_OK) return st;
+    if (!qkv || !k_cache || !v_cache || !cos || !sin || !pos || !out) return AWQ_ERR_NULL_POINTER;
+    if (!aligned(qkv, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(cos, 16) ||
+        !aligned(sin, 16) || !aligned(pos, 8) || !aligned(out, 2) || !aligned(workspace, 16))
+        return AWQ_ERR_MISALIGNED;
+    if (!workspace || workspace_bytes < decode_attn_workspace((int)max_seq, (int)num_heads, (int)head_dim))
+        return AWQ_ERR_WORKSPACE;
+    DecodeAttnArgs a;
+    a.qkv = static_cast<const half_t*>(qkv);
+    a.k_cache = static_cast<half_t*>(k_cache);
+    a.v_cache = static_cast<half_t*>(v_cache);
+    a.cos = static_cast<const float*>(cos);
+    a.sin = static_cast<const float*>(sin);
+    a.pos = pos;
+    a.part = static_cast<float*>(workspace);
+    a.out = static_cast<half_t*>(out);
+    a.nh = (int)num_heads;
+    a.kvh = (int)num_kv_heads;
+    a.max_seq = (int)max_seq;
+    const hipError_t e = launch_decode_attn(a, (int)head_dim, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
 }
 

@@ -76,6 +76,23 @@ int fp16_gemv_max_k();
 // out[m, i] = fp16(silu(gate_up[m, i]) * gate_up[m, I + i]); I % 8 == 0.
 hipError_t launch_silu_mul(const half_t* gate_up, half_t* out, int M, int I, hipStream_t stream);
 
+// One decode position's attention (awq_attention_decode.hip): head size 64 or 128,
+// nh a multiple of kvh; part: decode_attn_workspace() bytes, no state between
+// calls.
+struct DecodeAttnArgs {
+    const half_t* qkv;       // [(nh + 2 kvh) * hd]: the new position's fused projection
+    half_t* k_cache;         // [kvh, max_seq, hd]; row pos is written
+    half_t* v_cache;
+    const float* cos;        // [max_seq, hd]
+    const float* sin;
+    const int64_t* pos;      // [1], on the device
+    float* part;
+    half_t* out;             // [nh * hd]
+    int nh, kvh, max_seq;
+};
+size_t decode_attn_workspace(int max_seq, int nh, int hd);
+hipError_t launch_decode_attn(const DecodeAttnArgs& a, int hd, hipStream_t stream);
+
 hipError_t launch_dequant(const uint32_t* qweight, const uint32_t* qzeros, const half_t* scales,
                           half_t* w, int N, int K, hipStream_t stream);
 

@@ -5,10 +5,11 @@ Mirrors the reference model and engine (``model/qwen2.py``, ``model/config.py``,
 (no checkpoint exists offline): every linear layer is an AWQ int4 projection
 run by ``kernels.awq_gemm.awq_gemm_forward`` (fused QKV with the q/k/v biases,
 ``model/qwen2.py:79-85,104-113``; fused gate||up, ``:174-188``), the logits
-come from the fp16 lm_head GEMV (``kernels.lm_head``, ``:253,280``), and the
-non-GEMM work -- embedding, RMSNorm (``:15-22``), rotate-half RoPE
-(``kernels/rope.py:41-57``), GQA attention over a static KV cache -- is
-plain torch (attention in fp32 on contiguous operands).  The QKV bias and
+come from the fp16 lm_head GEMV (``kernels.lm_head``, ``:253,280``), RoPE
+(``kernels/rope.py:41-57``), the static KV cache's new row and the GQA
+attention of a decode step run in ``kernels.attention`` (head sizes 64 and
+128), and the rest -- embedding, RMSNorm (``:15-22``), the prefill's
+attention -- is plain torch (attention in fp32 on contiguous operands).  The QKV bias and
 the residual adds after o_proj and down_proj run in the GEMM's epilogue,
 and SiLU * up reads the fused gate||up output in one kernel
 (``kernels.silu_mul``).  Logits are computed for the last position only, where the
@@ -29,6 +30,7 @@ import time
 
 import torch
 
+from kernels.attention import attention_decode, attention_served
 from kernels.awq_gemm import awq_gemm_forward, awq_gemm_forward_ex
 from kernels.lm_head import lm_head_forward
 from kernels.silu_mul import silu_mul_gate_up
@@ -154,6 +156,8 @@ class Qwen2AwqDecoder:
         L, KV = shape.num_layers, shape.num_kv_heads
         self.k_cache = torch.zeros((L, KV, max_seq_len, hd), dtype=torch.float16, device=self.dev)
         self.v_cache = torch.zeros_like(self.k_cache)
+        # the HIP attention serves heads of 64 or 128 columns; torch the others
+        self._hip_attention = attention_served(shape.num_heads, KV, hd, max_seq_len)
         self._graph = None
 
     # ---- linear layers: the path this build replaces -------------------------
@@ -169,10 +173,22 @@ class Qwen2AwqDecoder:
     def _layer(self, li: int, h: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         s = self.s
         p = self.layers[li]
-        S = h.shape[0]
-        nh, kvh, hd = s.num_heads, s.num_kv_heads, s.head_dim
         x = _rmsnorm(h, p["ln1"], s.rms_norm_eps)
         qkv = self.linear(x, p["qkv"], bias=p["qkv_bias"])
+        att = self._attention(li, qkv, pos, causal)
+        h = self.linear(att, p["o"], residual=h)
+        x = _rmsnorm(h, p["ln2"], s.rms_norm_eps)
+        inter = silu_mul_gate_up(self.linear(x, p["gate_up"]))
+        return self.linear(inter, p["down"], residual=h)
+
+    def _attention(self, li: int, qkv: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
+        """Attention output fp16 [S, heads * head_dim] of the positions `pos`,
+        whose keys and values go into the layer's caches."""
+        s = self.s
+        S = qkv.shape[0]
+        nh, kvh, hd = s.num_heads, s.num_kv_heads, s.head_dim
+        if not causal and self._hip_attention:
+            return attention_decode(qkv, self.k_cache[li], self.v_cache[li], self.cos, self.sin, pos, nh)
         q = qkv[:, :nh * hd].view(S, nh, hd).float()
         k = qkv[:, nh * hd:(nh + kvh) * hd].view(S, kvh, hd).float()
         v = qkv[:, (nh + kvh) * hd:].view(S, kvh, hd)
@@ -199,11 +215,7 @@ class Qwen2AwqDecoder:
         scores = scores.view(kvh, groups, S, T).masked_fill(mask, float("-inf"))
         probs = torch.softmax(scores, dim=-1).view(kvh, groups * S, T)
         att = torch.matmul(probs, vv.contiguous()).view(nh, S, hd)            # [nh, S, hd]
-        att = att.transpose(0, 1).reshape(S, nh * hd).half()
-        h = self.linear(att, p["o"], residual=h)
-        x = _rmsnorm(h, p["ln2"], s.rms_norm_eps)
-        inter = silu_mul_gate_up(self.linear(x, p["gate_up"]))
-        return self.linear(inter, p["down"], residual=h)
+        return att.transpose(0, 1).reshape(S, nh * hd).half()
 
     def _forward(self, ids: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         h = torch.nn.functional.embedding(ids, self.embed)
@@ -225,6 +237,8 @@ class Qwen2AwqDecoder:
     @torch.no_grad()
     def decode_logits(self, token: torch.Tensor, pos: int) -> torch.Tensor:
         """One eager decode step: logits after feeding `token` at position `pos`."""
+        if not 0 <= pos < self.max_seq_len:
+            raise ValueError(f"position {pos} outside [0, {self.max_seq_len})")
         return self._forward(token.view(1).to(self.dev), torch.tensor([pos], device=self.dev), causal=False)
 
     @torch.no_grad()

@@ -1,0 +1,102 @@
+"""The engine's attention kernels (``kernels/attention.py``) against the same
+attention in 64 bits, in plain torch on the CPU.
+
+Bound per element: one fp16 rounding of the result (2^-11 of it, or half of
+the smallest subnormal), and for the fp32 work before it 2e-5 of the largest
+value: a dot product of d terms and a sum over T positions err by a few of
+their square roots times 2^-24 (d = 128, T = 2000: about 3e-6), and an error e
+of a score moves its probability by e, scores being up to about 20.
+"""
+import math
+
+import pytest
+import torch
+
+from kernels import _native
+from kernels.attention import attention_decode, attention_served
+
+pytestmark = pytest.mark.gpu
+
+
+def _tables(max_seq, hd, dev):
+    inv = 1.0 / (1e6 ** (torch.arange(0, hd, 2, dtype=torch.float32) / hd))
+    f = torch.outer(torch.arange(max_seq, dtype=torch.float32), inv)
+    f = torch.cat((f, f), -1)
+    return f.cos().to(dev), f.sin().to(dev)
+
+
+def _rope64(t, cos, sin):
+    """t [S, heads, hd] in 64 bits; cos, sin [S, hd]."""
+    h = t.shape[-1] // 2
+    return t * cos.unsqueeze(1) + torch.cat((-t[..., h:], t[..., :h]), -1) * sin.unsqueeze(1)
+
+
+def _attend64(q, k, v, first):
+    """q [S, nh, hd] of positions first .., k and v [kvh, T, hd]: [S, nh * hd]."""
+    S, nh, hd = q.shape
+    out = torch.empty((S, nh, hd), dtype=torch.float64)
+    mask = torch.arange(k.shape[1]).unsqueeze(0) > torch.arange(first, first + S).unsqueeze(1)
+    for h in range(nh):
+        g = h // (nh // k.shape[0])
+        s = (q[:, h] @ k[g].t().contiguous() / math.sqrt(hd)).masked_fill(mask, float("-inf"))
+        out[:, h] = torch.softmax(s, -1) @ v[g]
+    return out.view(S, nh * hd)
+
+
+def _close(y, ref, what):
+    y = y.double().cpu()
+    bound = ref.abs() * 2.0**-11 + 2.0**-25 + 2e-5 * ref.abs().max()
+    worst = ((y - ref).abs() / bound).max().item()
+    assert torch.isfinite(y).all() and worst <= 1.0, f"{what}: {worst:.2f} of the bound"
+
+
+@pytest.mark.parametrize("nh,kvh,hd,max_seq,positions", [
+    (28, 4, 128, 1152, (0, 1, 15, 16, 63, 64, 65, 1023, 1151)),
+    (28, 4, 128, 5000, (127, 128, 4095, 4999)),        # ranges of 128 positions
+    (4, 2, 64, 64, (0, 7, 63)),
+    (6, 2, 64, 130, (128, 129)),
+    (12, 1, 64, 100, (99,)),                           # more query heads than one workgroup takes
+    (3, 3, 128, 1, (0,)),
+    (18, 2, 128, 70, (64, 69)),
+])
+def test_attention_decode(gpu, nh, kvh, hd, max_seq, positions):
+    g = torch.Generator().manual_seed(max_seq)
+    cos, sin = _tables(max_seq, hd, gpu)
+    k0 = torch.randn((kvh, max_seq, hd), generator=g).half()
+    v0 = torch.randn((kvh, max_seq, hd), generator=g).half()
+    for pos in positions:
+        print(f"attention_decode nh={nh} kvh={kvh} hd={hd} max_seq={max_seq} pos={pos}", flush=True)
+        qkv = (torch.randn((1, (nh + 2 * kvh) * hd), generator=g) * 2).half()
+        kc, vc = k0.to(gpu), v0.to(gpu)
+        kc[:, pos + 1:] = float("nan")                 # rows past the position are never used
+        vc[:, pos + 1:] = float("nan")
+        keep_k, keep_v = kc.clone(), vc.clone()
+        out = attention_decode(qkv.to(gpu), kc, vc, cos, sin, torch.tensor([pos], device=gpu), nh)
+        c, s = cos[pos:pos + 1].cpu().double(), sin[pos:pos + 1].cpu().double()
+        heads = qkv.double().view(1, nh + 2 * kvh, hd)
+        q, knew = _rope64(heads[:, :nh], c, s), _rope64(heads[:, nh:nh + kvh], c, s)
+        k, v = k0[:, :pos + 1].double(), v0[:, :pos + 1].double()
+        v[:, pos] = heads[0, nh + kvh:]
+        _close(kc[:, pos], knew[0], "new key")
+        k[:, pos] = kc[:, pos].double().cpu()          # the cache holds fp16 keys
+        assert torch.equal(vc[:, pos].cpu(), v[:, pos].half())
+        keep_k[:, pos], keep_v[:, pos] = kc[:, pos], vc[:, pos]
+        assert torch.equal(kc.view(torch.int16), keep_k.view(torch.int16))
+        assert torch.equal(vc.view(torch.int16), keep_v.view(torch.int16))
+        _close(out, _attend64(q, k, v, pos), "attention")
+
+
+def test_attention_decode_refuses(gpu):
+    cos, sin = _tables(8, 64, gpu)
+    c = torch.zeros((2, 8, 64), dtype=torch.float16, device=gpu)
+    qkv = torch.zeros((1, 8 * 64), dtype=torch.float16, device=gpu)
+    pos = torch.zeros(1, dtype=torch.int64, device=gpu)
+    attention_decode(qkv, c, c.clone(), cos, sin, pos, 4)
+    for bad in (dict(qkv=qkv.float()), dict(qkv=qkv[:, :-64]), dict(pos=pos.int()), dict(cos=cos[:4]),
+                dict(k_cache=c.transpose(0, 1)), dict(k_cache=c[:1])):
+        args = dict(qkv=qkv, k_cache=c, v_cache=c.clone(), cos=cos, sin=sin, pos=pos) | bad
+        with pytest.raises(ValueError):
+            attention_decode(num_heads=4, **args)
+    with pytest.raises(_native.AwqNativeError):        # head counts that do not divide
+        attention_decode(torch.zeros((1, 7 * 64), dtype=torch.float16, device=gpu), c, c.clone(), cos, sin, pos, 3)
+    assert attention_served(28, 4, 128, 2048) and not attention_served(4, 2, 32, 64)
