@@ -340,6 +340,19 @@ int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, con
                               int64_t head_dim, int64_t max_seq, void* workspace, size_t workspace_bytes,
                               void* stream);
 
+/* Causal attention of a prompt's positions 0 .. S - 1 (the prefill of
+ * model/qwen2.py:104-163): as awq_fp16_attention_decode for every position,
+ * with rows 0 .. S - 1 of the caches written.  qkv fp16 [S, (num_heads + 2
+ * num_kv_heads) * head_dim], out fp16 [S, num_heads * head_dim], S <= max_seq;
+ * S == 0 is a valid no-op.  q and the probabilities enter the matrix cores as
+ * sums of two fp16 values (22 bits), with fp32 sums.  workspace: at least
+ * awq_fp16_attention_prefill_workspace bytes, of any content; it holds nothing
+ * between calls.  Two launches. */
+size_t awq_fp16_attention_prefill_workspace(int64_t S, int64_t num_kv_heads, int64_t head_dim);
+int awq_fp16_attention_prefill(const void* qkv, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                               void* out, int64_t S, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                               int64_t max_seq, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1206,4 +1206,39 @@ int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, con
     return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
 }
 
+size_t awq_fp16_attention_prefill_workspace(int64_t S, int64_t num_kv_heads, int64_t head_dim) {
+    if (S <= 0 || check_attention(num_kv_heads, num_kv_heads, head_dim, S) != AWQ_OK) return 0;
+    return prefill_attn_workspace((int)S, (int)num_kv_heads, (int)head_dim);
+}
+
+int awq_fp16_attention_prefill(const void* qkv, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                               void* out, int64_t S, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                               int64_t max_seq, void* workspace, size_t workspace_bytes, void* stream) {
+    const int st = check_attention(num_heads, num_kv_heads, head_dim, max_seq);
+    if (st != AWQ_OK) return st;
+    if (S < 0 || S > max_seq) return AWQ_ERR_BAD_DIMS;
+    if (S > kIndexLimit / num_heads) return AWQ_ERR_TOO_LARGE;   // one workgroup per head and 64 positions
+    if (S == 0) return AWQ_OK;
+    if (!qkv || !k_cache || !v_cache || !cos || !sin || !out) return AWQ_ERR_NULL_POINTER;
+    if (!aligned(qkv, 16) || !aligned(k_cache, 16) || !aligned(v_cache, 16) || !aligned(cos, 16) ||
+        !aligned(sin, 16) || !aligned(out, 8) || !aligned(workspace, 16))
+        return AWQ_ERR_MISALIGNED;
+    if (!workspace || workspace_bytes < prefill_attn_workspace((int)S, (int)num_kv_heads, (int)head_dim))
+        return AWQ_ERR_WORKSPACE;
+    PrefillAttnArgs a;
+    a.qkv = static_cast<const half_t*>(qkv);
+    a.k_cache = static_cast<half_t*>(k_cache);
+    a.v_cache = static_cast<half_t*>(v_cache);
+    a.cos = static_cast<const float*>(cos);
+    a.sin = static_cast<const float*>(sin);
+    a.vt = static_cast<half_t*>(workspace);
+    a.out = static_cast<half_t*>(out);
+    a.S = (int)S;
+    a.nh = (int)num_heads;
+    a.kvh = (int)num_kv_heads;
+    a.max_seq = (int)max_seq;
+    const hipError_t e = launch_prefill_attn(a, (int)head_dim, (int)cus(), static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
+}
+
 }  // extern "C"

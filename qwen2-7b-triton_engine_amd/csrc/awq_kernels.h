@@ -90,6 +90,20 @@ struct DecodeAttnArgs {
     half_t* out;             // [nh * hd]
     int nh, kvh, max_seq;
 };
+// A prompt's causal attention (awq_attention_prefill.hip): positions 0 .. S - 1,
+// S <= max_seq; vt: prefill_attn_workspace() bytes, no state between calls.
+struct PrefillAttnArgs {
+    const half_t* qkv;       // [S, (nh + 2 kvh) * hd]
+    half_t* k_cache;         // [kvh, max_seq, hd]; rows 0 .. S - 1 are written
+    half_t* v_cache;
+    const float* cos;        // [max_seq, hd]
+    const float* sin;
+    half_t* vt;
+    half_t* out;             // [S, nh * hd]
+    int S, nh, kvh, max_seq;
+};
+size_t prefill_attn_workspace(int S, int kvh, int hd);
+hipError_t launch_prefill_attn(const PrefillAttnArgs& a, int hd, int cus, hipStream_t stream);
 size_t decode_attn_workspace(int max_seq, int nh, int hd);
 hipError_t launch_decode_attn(const DecodeAttnArgs& a, int hd, hipStream_t stream);
 

@@ -7,9 +7,9 @@ run by ``kernels.awq_gemm.awq_gemm_forward`` (fused QKV with the q/k/v biases,
 ``model/qwen2.py:79-85,104-113``; fused gate||up, ``:174-188``), the logits
 come from the fp16 lm_head GEMV (``kernels.lm_head``, ``:253,280``), RoPE
 (``kernels/rope.py:41-57``), the static KV cache's new row and the GQA
-attention of a decode step run in ``kernels.attention`` (head sizes 64 and
-128), and the rest -- embedding, RMSNorm (``:15-22``), the prefill's
-attention -- is plain torch (attention in fp32 on contiguous operands).  The QKV bias and
+attention run in ``kernels.attention`` (head sizes 64 and 128; other sizes
+in torch, in fp32 on contiguous operands), and the rest -- embedding, RMSNorm
+(``:15-22``) -- is plain torch.  The QKV bias and
 the residual adds after o_proj and down_proj run in the GEMM's epilogue,
 and SiLU * up reads the fused gate||up output in one kernel
 (``kernels.silu_mul``).  Logits are computed for the last position only, where the
@@ -30,7 +30,7 @@ import time
 
 import torch
 
-from kernels.attention import attention_decode, attention_served
+from kernels.attention import attention_decode, attention_prefill, attention_served
 from kernels.awq_gemm import awq_gemm_forward, awq_gemm_forward_ex
 from kernels.lm_head import lm_head_forward
 from kernels.silu_mul import silu_mul_gate_up
@@ -187,8 +187,11 @@ class Qwen2AwqDecoder:
         s = self.s
         S = qkv.shape[0]
         nh, kvh, hd = s.num_heads, s.num_kv_heads, s.head_dim
-        if not causal and self._hip_attention:
-            return attention_decode(qkv, self.k_cache[li], self.v_cache[li], self.cos, self.sin, pos, nh)
+        if self._hip_attention:
+            k_cache, v_cache = self.k_cache[li], self.v_cache[li]
+            if causal:
+                return attention_prefill(qkv, k_cache, v_cache, self.cos, self.sin, nh)
+            return attention_decode(qkv, k_cache, v_cache, self.cos, self.sin, pos, nh)
         q = qkv[:, :nh * hd].view(S, nh, hd).float()
         k = qkv[:, nh * hd:(nh + kvh) * hd].view(S, kvh, hd).float()
         v = qkv[:, (nh + kvh) * hd:].view(S, kvh, hd)

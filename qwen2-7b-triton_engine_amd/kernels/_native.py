@@ -94,6 +94,9 @@ SIGNATURES = {
     "awq_fp16_attention_decode_workspace": (ctypes.c_size_t, [_I64, _I64, _I64, _I64]),
     "awq_fp16_attention_decode": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _VP,
                                                  ctypes.c_size_t, _VP]),
+    "awq_fp16_attention_prefill_workspace": (ctypes.c_size_t, [_I64, _I64, _I64]),
+    "awq_fp16_attention_prefill": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _I64, _VP,
+                                                  ctypes.c_size_t, _VP]),
     "awq_w4a16_gemm_noalloc": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I32, _VP]),
 }
 

@@ -3,7 +3,8 @@
 ``attention_decode`` is one new position over a static KV cache, from the
 fused QKV projection to the attention output: RoPE, the cache's new row,
 softmax(q K^T / sqrt(d)) V in fp32 (``model/qwen2.py:104-163``,
-``kernels/rope.py:41-57``) -- two launches.
+``kernels/rope.py:41-57``) -- two launches.  ``attention_prefill`` is the same
+for a prompt's positions 0 .. S - 1.
 """
 from __future__ import annotations
 
@@ -12,7 +13,7 @@ import torch
 from . import _native
 from .awq_gemm import _OnDevice, _stream_handle
 
-__all__ = ["attention_decode", "attention_served"]
+__all__ = ["attention_decode", "attention_prefill", "attention_served"]
 
 
 def attention_served(num_heads: int, num_kv_heads: int, head_dim: int, max_seq: int) -> bool:
@@ -53,4 +54,28 @@ def attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
                                          sin.data_ptr(), pos.data_ptr(), out.data_ptr(), num_heads, kvh, hd, max_seq,
                                          ws.data_ptr(), ws.numel(), _stream_handle(dev))
     _native.check(st, "awq_fp16_attention_decode")
+    return out
+
+
+def attention_prefill(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, cos: torch.Tensor,
+                      sin: torch.Tensor, num_heads: int) -> torch.Tensor:
+    """Causal attention fp16 ``[S, num_heads * head_dim]`` of positions 0 .. S - 1
+    (``qkv`` fp16 ``[S, (num_heads + 2 kv_heads) * head_dim]``); their k and v go
+    into the first S rows of the caches."""
+    dev = qkv.device
+    kvh, max_seq, hd = _check_cache(dev, k_cache, v_cache, cos, sin)
+    if qkv.dtype != torch.float16 or qkv.dim() != 2 or qkv.shape[1] != (num_heads + 2 * kvh) * hd \
+            or not qkv.is_contiguous():
+        raise ValueError(f"qkv must be a contiguous fp16 tensor [S, {(num_heads + 2 * kvh) * hd}]")
+    S = qkv.shape[0]
+    if S > max_seq:
+        raise ValueError(f"{S} positions exceed the cache's {max_seq}")
+    L = _native.lib()
+    ws = torch.empty(L.awq_fp16_attention_prefill_workspace(S, kvh, hd), dtype=torch.uint8, device=dev)
+    out = torch.empty((S, num_heads * hd), dtype=torch.float16, device=dev)
+    with _OnDevice(dev):
+        st = L.awq_fp16_attention_prefill(qkv.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cos.data_ptr(),
+                                          sin.data_ptr(), out.data_ptr(), S, num_heads, kvh, hd, max_seq,
+                                          ws.data_ptr(), ws.numel(), _stream_handle(dev))
+    _native.check(st, "awq_fp16_attention_prefill")
     return out

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from kernels import _native
-from kernels.attention import attention_decode, attention_served
+from kernels.attention import attention_decode, attention_prefill, attention_served
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +84,53 @@ def test_attention_decode(gpu, nh, kvh, hd, max_seq, positions):
         assert torch.equal(kc.view(torch.int16), keep_k.view(torch.int16))
         assert torch.equal(vc.view(torch.int16), keep_v.view(torch.int16))
         _close(out, _attend64(q, k, v, pos), "attention")
+
+
+@pytest.mark.parametrize("nh,kvh,hd,max_seq,lengths", [
+    (28, 4, 128, 1200, (1, 2, 15, 17, 63, 64, 65, 127, 129, 700, 1153)),
+    (4, 2, 64, 700, (1, 33, 64, 200, 700)),
+    (128, 2, 64, 840, (833,)),                          # 128 queries per workgroup
+    (128, 2, 128, 790, (769,)),
+    (3, 3, 128, 70, (70,)),
+])
+def test_attention_prefill(gpu, nh, kvh, hd, max_seq, lengths):
+    g = torch.Generator().manual_seed(max_seq + 1)
+    cos, sin = _tables(max_seq, hd, gpu)
+    for S in lengths:
+        print(f"attention_prefill nh={nh} kvh={kvh} hd={hd} max_seq={max_seq} S={S}", flush=True)
+        qkv = (torch.randn((S, (nh + 2 * kvh) * hd), generator=g) * 2).half()
+        kc = torch.full((kvh, max_seq, hd), float("nan"), dtype=torch.float16, device=gpu)
+        vc = kc.clone()
+        out = attention_prefill(qkv.to(gpu), kc, vc, cos, sin, nh)
+        c, s = cos[:S].cpu().double(), sin[:S].cpu().double()
+        heads = qkv.double().view(S, nh + 2 * kvh, hd)
+        q, knew = _rope64(heads[:, :nh], c, s), _rope64(heads[:, nh:nh + kvh], c, s)
+        _close(kc[:, :S], knew.transpose(0, 1), "keys")
+        v = heads[:, nh + kvh:].transpose(0, 1)
+        assert torch.equal(vc[:, :S].cpu().double(), v)
+        assert kc[:, S:].isnan().all() and vc[:, S:].isnan().all()
+        _close(out, _attend64(q, kc[:, :S].double().cpu(), v, 0), "attention")
+
+
+def test_attention_prefill_and_decode_agree_on_extremes(gpu):
+    """Values from 1e-4 to 2, queries of one sign: the split operands keep
+    their bits, and a position's attention is the same from both kernels."""
+    nh, kvh, hd, S = 8, 2, 128, 190
+    cos, sin = _tables(S, hd, gpu)
+    g = torch.Generator().manual_seed(5)
+    for scale in (1e-4, 1e-2, 1.0, 2.0):
+        print(f"attention extremes: scale {scale}", flush=True)
+        qkv = (torch.randn((S, (nh + 2 * kvh) * hd), generator=g) * scale).half()
+        qkv[:, :nh * hd] += torch.tensor(scale).half()
+        kc = torch.zeros((kvh, S, hd), dtype=torch.float16, device=gpu)
+        vc = kc.clone()
+        out = attention_prefill(qkv.to(gpu), kc, vc, cos, sin, nh)
+        c, s = cos.cpu().double(), sin.cpu().double()
+        heads = qkv.double().view(S, nh + 2 * kvh, hd)
+        ref = _attend64(_rope64(heads[:, :nh], c, s), kc.double().cpu(), heads[:, nh + kvh:].transpose(0, 1), 0)
+        _close(out, ref, "prefill")
+        one = attention_decode(qkv[-1:].contiguous().to(gpu), kc, vc, cos, sin, torch.tensor([S - 1], device=gpu), nh)
+        _close(one, ref[-1:], "decode")
 
 
 def test_attention_decode_refuses(gpu):
