@@ -322,6 +322,11 @@ int awq_silu_mul(const void* gate_up, void* out, int64_t M, int64_t I, void* str
 int awq_fp16_linear(const void* x, const void* weight, void* out, int64_t M, int64_t N, int64_t K,
                     void* stream);
 
+/* out[m] = fp16(x[m] * rsqrt(mean(x[m]^2) + eps) * w) in fp32, rounded once:
+ * the RMSNorm of model/qwen2.py:15-22.  x and out fp16 [M, H], w fp16 [H], all
+ * 16-byte aligned; H % 8 == 0, H <= 16384 (AWQ_ERR_PATH above). */
+int awq_fp16_rmsnorm(const void* x, const void* w, void* out, int64_t M, int64_t H, float eps, void* stream);
+
 /* Attention of one new position over a static KV cache (the decode step of
  * model/qwen2.py:104-163): rotate-half RoPE of q and k (fp32), k (rounded to
  * fp16) and v stored at row *pos of the caches, softmax(q K^T / sqrt(head_dim))

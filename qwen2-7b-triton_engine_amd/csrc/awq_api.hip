@@ -1172,6 +1172,19 @@ int awq_fp16_linear(const void* x, const void* weight, void* out, int64_t M, int
     return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
 }
 
+int awq_fp16_rmsnorm(const void* x, const void* w, void* out, int64_t M, int64_t H, float eps, void* stream) {
+    if (M < 0 || H <= 0 || H % 8 != 0) return AWQ_ERR_BAD_DIMS;
+    if (H > rmsnorm_max_h()) return AWQ_ERR_PATH;
+    if (M > kIndexLimit) return AWQ_ERR_TOO_LARGE;
+    if (M == 0) return AWQ_OK;
+    if (!x || !w || !out) return AWQ_ERR_NULL_POINTER;
+    if (!aligned(x, 16) || !aligned(w, 16) || !aligned(out, 16)) return AWQ_ERR_MISALIGNED;
+    const hipError_t e = launch_rmsnorm(static_cast<const half_t*>(x), static_cast<const half_t*>(w),
+                                        static_cast<half_t*>(out), (int)M, (int)H, eps,
+                                        static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
+}
+
 size_t awq_fp16_attention_decode_workspace(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
                                            int64_t max_seq) {
     if (check_attention(num_heads, num_kv_heads, head_dim, max_seq) != AWQ_OK) return 0;

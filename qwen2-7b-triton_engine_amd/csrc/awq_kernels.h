@@ -76,6 +76,11 @@ int fp16_gemv_max_k();
 // out[m, i] = fp16(silu(gate_up[m, i]) * gate_up[m, I + i]); I % 8 == 0.
 hipError_t launch_silu_mul(const half_t* gate_up, half_t* out, int M, int I, hipStream_t stream);
 
+// out[m] = fp16(x[m] * rsqrt(mean(x[m]^2) + eps) * w); H % 8 == 0, H <=
+// rmsnorm_max_h().
+hipError_t launch_rmsnorm(const half_t* x, const half_t* w, half_t* out, int M, int H, float eps, hipStream_t stream);
+int rmsnorm_max_h();
+
 // One decode position's attention (awq_attention_decode.hip): head size 64 or 128,
 // nh a multiple of kvh; part: decode_attn_workspace() bytes, no state between
 // calls.

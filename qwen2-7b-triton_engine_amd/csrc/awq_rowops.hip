@@ -1,0 +1,78 @@
+// Row operations of the Qwen2 engine between its projections: RMSNorm.
+#include "awq_kernels.h"
+
+namespace awq {
+namespace {
+
+constexpr int kNormThreads = 512;
+
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+    for (int w = 1; w < 64; w *= 2) v += __shfl_xor(v, w);
+    return v;
+}
+
+// out[m] = fp16(x[m] * rsqrt(mean(x[m]^2) + eps) * w) in fp32
+// (model/qwen2.py:15-22).  One workgroup per row, C 16-byte pieces of it per
+// thread held in registers between the sum and the store: the row is read
+// once.  Bound by latency at decode (one load, one cross-wave sum, one
+// store), by memory over a prompt.  The torch form was five launches and as
+// many passes over fp32 copies of the row: with it a token of a 28-layer model
+// took 1.3 ms more, and a 1777-token prefill of four layers 4.36 ms against
+// 3.89 now.
+template <int C>
+__global__ __launch_bounds__(kNormThreads) void awq_rmsnorm_kernel(const half_t* __restrict__ x,
+                                                                   const half_t* __restrict__ w,
+                                                                   half_t* __restrict__ out, int H, float eps) {
+    __shared__ float sums[kNormThreads / 64];
+    const int pieces = H / 8;
+    const half8_t* xr = reinterpret_cast<const half8_t*>(x + (size_t)blockIdx.x * H);
+    const half8_t* wr = reinterpret_cast<const half8_t*>(w);
+    half8_t v[C], g[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int i = c * kNormThreads + threadIdx.x;
+        v[c] = half8_t{};
+        g[c] = half8_t{};
+        if (i < pieces) {
+            v[c] = xr[i];
+            g[c] = wr[i];
+        }
+    }
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = fmaf((float)v[c][e], (float)v[c][e], s);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kNormThreads / 64; ++i) s += sums[i];
+    const float r = 1.0f / sqrtf(s / (float)H + eps);
+    half8_t* orow = reinterpret_cast<half8_t*>(out + (size_t)blockIdx.x * H);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int i = c * kNormThreads + threadIdx.x;
+        if (i >= pieces) continue;
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (half_t)((float)v[c][e] * r * (float)g[c][e]);
+        orow[i] = o;
+    }
+}
+
+}  // namespace
+
+int rmsnorm_max_h() { return 4 * kNormThreads * 8; }
+
+hipError_t launch_rmsnorm(const half_t* x, const half_t* w, half_t* out, int M, int H, float eps, hipStream_t stream) {
+    if (M == 0) return hipSuccess;
+    const int c = (H / 8 + kNormThreads - 1) / kNormThreads;
+    auto kernel = c <= 1 ? awq_rmsnorm_kernel<1> : c <= 2 ? awq_rmsnorm_kernel<2> : awq_rmsnorm_kernel<4>;
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, H, eps);
+    return hipGetLastError();
+}
+
+}  // namespace awq

@@ -8,8 +8,8 @@ run by ``kernels.awq_gemm.awq_gemm_forward`` (fused QKV with the q/k/v biases,
 come from the fp16 lm_head GEMV (``kernels.lm_head``, ``:253,280``), RoPE
 (``kernels/rope.py:41-57``), the static KV cache's new row and the GQA
 attention run in ``kernels.attention`` (head sizes 64 and 128; other sizes
-in torch, in fp32 on contiguous operands), and the rest -- embedding, RMSNorm
-(``:15-22``) -- is plain torch.  The QKV bias and
+in torch, in fp32 on contiguous operands), RMSNorm (``:15-22``) in
+``kernels.rmsnorm``, and the embedding lookup in torch.  The QKV bias and
 the residual adds after o_proj and down_proj run in the GEMM's epilogue,
 and SiLU * up reads the fused gate||up output in one kernel
 (``kernels.silu_mul``).  Logits are computed for the last position only, where the
@@ -33,6 +33,7 @@ import torch
 from kernels.attention import attention_decode, attention_prefill, attention_served
 from kernels.awq_gemm import awq_gemm_forward, awq_gemm_forward_ex
 from kernels.lm_head import lm_head_forward
+from kernels.rmsnorm import MAX_H, rmsnorm
 from kernels.silu_mul import silu_mul_gate_up
 
 __all__ = ["Qwen2Shape", "QWEN2_7B", "Qwen2AwqDecoder"]
@@ -69,6 +70,8 @@ def _awq_tensors(k: int, n: int, gen: torch.Generator, dev: torch.device):
 
 
 def _rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    if x.dtype == w.dtype == torch.float16 and w.dim() == 1 and x.shape[-1] <= MAX_H and x.is_cuda:
+        return rmsnorm(x, w, eps)        # hidden sizes are multiples of the 128-row group
     xf = x.float()
     return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps) * w.float()).half()
 

@@ -91,6 +91,7 @@ SIGNATURES = {
     "awq_w4a16_gemm_epilogue": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I32, _VP,
                                                ctypes.c_size_t, ctypes.POINTER(Plan), _VP]),
     "awq_silu_mul": (ctypes.c_int, [_VP, _VP, _I64, _I64, _VP]),
+    "awq_fp16_rmsnorm": (ctypes.c_int, [_VP, _VP, _VP, _I64, _I64, ctypes.c_float, _VP]),
     "awq_fp16_attention_decode_workspace": (ctypes.c_size_t, [_I64, _I64, _I64, _I64]),
     "awq_fp16_attention_decode": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _VP,
                                                  ctypes.c_size_t, _VP]),
