@@ -1,8 +1,8 @@
 // Decode attention of the Qwen2 engine: one new position against a static KV
 // cache, from the fused QKV projection to the attention output
 // (model/qwen2.py:104-163: rotate-half RoPE, cache update, GQA softmax
-// attention).  fp16 operands, every product and sum in fp32; q stays fp32
-// after RoPE, the probabilities stay fp32.
+// attention).  q after RoPE and the probabilities are fp32 values, summed in
+// fp32.
 //
 // What bounds it: latency.  A thousand positions of 4 KV heads are 2 MB, a
 // third of a microsecond of HBM time; the torch form of the same step read
@@ -10,197 +10,197 @@
 // Here it is two launches: the cache is split along its positions over
 // enough workgroups to load it at once, each keeps a running softmax of its
 // range for all query heads of one KV head (so K and V are read once), and a
-// second launch weights the ranges' partial sums.  Measured on Qwen2-7B: a
-// 1024-token prompt and 48 greedy tokens, 28 layers, cache of 1152 positions,
-// 301 -> 190 ms (2.3 ms less per token); eight eager steps of a 4-layer stack
-// at position 900 of 2048, 13.9 -> 6.9 ms.
+// second launch weights the ranges' partial sums.  Measured on Qwen2-7B's
+// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 10.2 us
+// for the two at position 1100, 8.1 of it the first -- a form of it with the
+// scores, the softmax and P V on the vector unit, 16 lanes a key, took 15.3.
 #include "awq_kernels.h"
 
 namespace awq {
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
-constexpr int kKeys = 64;   // positions of one inner pass of a workgroup: 16 per wave
+constexpr int kHeads = 16;             // query heads of one workgroup: the columns of an MFMA
+constexpr int kKeys = 16 * kWaves;     // positions of one inner pass of a workgroup: 16 per wave
+constexpr float kQScale = 4.0f;        // see split16
+constexpr float kPExp = 14.0f;
 
-// Sum over aligned groups of 16 (8) lanes, left in every lane: rotations
-// within a 16-lane DPP row (within its halves: mirror, quad permutations).
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-template <int LANES>
-__device__ __forceinline__ float group_sum(float v) {
-    v += dpp<0xB1>(v);    // quad_perm [1,0,3,2]
-    v += dpp<0x4E>(v);    // quad_perm [2,3,0,1]
-    v += dpp<0x141>(v);   // row_half_mirror: lane i <-> 7 - i
-    if (LANES == 16) v += dpp<0x140>(v);   // row_mirror: lane i <-> 15 - i
-    return v;
-}
-
-__device__ __forceinline__ float rope(float x, float partner, float c, float s, bool low) {
-    return x * c + (low ? -partner : partner) * s;
+// x = hi + lo in two fp16 values, 22 bits while lo stays above fp16's
+// smallest steps: q is scaled by 4 and the probabilities by 2^14 before the
+// split, powers of two that cancel exactly.  x is made opaque first: the
+// compiler would otherwise round the product that x is straight to fp16 for
+// one use of hi and by way of fp32 for the other.
+template <int N, typename V>
+__device__ __forceinline__ void split16(float (&x)[N], V& hi, V& lo) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        asm("" : "+v"(x[e]));
+        hi[e] = (half_t)x[e];
+        lo[e] = (half_t)(x[e] - (float)hi[e]);
+    }
 }
 
-// One workgroup: positions [split * chunk, ...) of one KV head for up to G
-// query heads.  Within an inner pass of 64 positions each wave owns 16: its
-// 16-lane (head size 64: 8-lane) groups each read one K row per load, 16 bytes
-// a lane, and reduce the dot products within the group; the wave's own 16
-// positions then go through its running softmax and its P V product, where
-// a lane owns HD / 64 columns of V.  The four waves' results meet once, at
+// One workgroup: positions [split * chunk, ...) of one KV head for up to 16
+// query heads, 16 positions per wave and pass.  S^T = K Q^T on the MFMA: its
+// columns are the heads, so one exponential covers four positions of every
+// head, and the result is already the B operand of O^T = V^T P^T (16x16x16).
+// V's row order in that product is free, so lane i takes columns i VC ..
+// i VC + VC - 1 of a V row with one load and supplies one of them to each of
+// VC products.  q and the probabilities are fp32 values split in two fp16
+// parts.  K, V and q are loaded before the position is known (rows of the
+// cache past it are masked), so the chain is two memory latencies long: the
+// position, then the RoPE row it selects.  The waves' results meet once, at
 // the end.
-template <int HD, int G>
+template <int HD>
 __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
-    const half_t* __restrict__ qkv, half_t* __restrict__ kc, half_t* __restrict__ vc, const float* __restrict__ cosp,
+    const half_t* __restrict__ qkv, half_t* kc, half_t* vc, const float* __restrict__ cosp,
     const float* __restrict__ sinp, const int64_t* __restrict__ posp, float* __restrict__ part, int nh, int kvh,
     int groups, int max_seq, int chunk) {
-    constexpr int kLpk = HD / 8;            // lanes per K row
-    constexpr int kRows = 64 / kLpk;        // K rows per load of a wave
-    constexpr int kPass = 16 / kRows;       // loads per 16 positions
-    constexpr int kVc = HD / 64;            // V columns per lane
-    typedef half_t vcols_t __attribute__((ext_vector_type(kVc)));
-    __shared__ __align__(16) float p_lds[kWaves][16][G];
-    __shared__ float m_lds[kWaves][G], l_lds[kWaves][G];
-    __shared__ float o_lds[kWaves][G][HD];
+    constexpr int kSteps = HD / 32;
+    constexpr int VC = HD / 16;            // V columns per lane
+    constexpr int kStride = HD + 4;        // floats per head of the reduction buffer
+    typedef half_t vcols_t __attribute__((ext_vector_type(VC)));
+    __shared__ float m_lds[kWaves][kHeads], l_lds[kWaves][kHeads];
+    __shared__ __align__(16) float o_lds[kWaves][kHeads][kStride];
 
-    const int64_t pos64 = *posp;
     const int split = blockIdx.x, g = blockIdx.y;
-    const int h0 = blockIdx.z * G;                       // first query head of this block within the group
-    const int heads = groups - h0 < G ? groups - h0 : G;
-    if (pos64 < 0 || pos64 >= max_seq || (int64_t)split * chunk > pos64) return;
-    const int pos = (int)pos64;
+    const int h0 = blockIdx.z * kHeads;    // first query head of this block within the group
+    const int heads = groups - h0 < kHeads ? groups - h0 : kHeads;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, t = lane >> 4;
     const int start = split * chunk;
-    const int end = start + chunk < pos + 1 ? start + chunk : pos + 1;
+    const int64_t pos64 = *posp;
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int sub = lane % kLpk, kr = lane / kLpk;
-    const int d0 = 8 * sub, dp = d0 < HD / 2 ? d0 + HD / 2 : d0 - HD / 2;
-    const bool low = d0 < HD / 2;
     half_t* kbase = kc + (size_t)g * max_seq * HD;
     half_t* vbase = vc + (size_t)g * max_seq * HD;
-    const half_t* knew = qkv + (size_t)nh * HD + (size_t)g * HD;
+    const half_t* qh = qkv + (size_t)(g * groups + h0 + (col < heads ? col : 0)) * HD;
+    const half_t* knew = qkv + (size_t)(nh + g) * HD;
     const half_t* vnew = knew + (size_t)kvh * HD;
-
-    half8_t kraw[kPass];
-    float vraw[16][kVc];
-    auto load = [&](int first) {   // rows past the last position are not read
+    half8_t kf[kSteps];
+    vcols_t vf[4];
+    auto load = [&](int first) {
+        const int krow = first + 16 * wave + col;
+        const half_t* ks = kbase + (size_t)(krow < max_seq ? krow : max_seq - 1) * HD + 8 * t;
 #pragma unroll
-        for (int i = 0; i < kPass; ++i) {
-            const int key = first + 16 * wave + i * kRows + kr;
-            kraw[i] = half8_t{};
-            if (key < end && key != pos) kraw[i] = *reinterpret_cast<const half8_t*>(kbase + (size_t)key * HD + d0);
-        }
+        for (int st = 0; st < kSteps; ++st) kf[st] = *reinterpret_cast<const half8_t*>(ks + 32 * st);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int key = first + 16 * wave + j;
-            const half_t* row = (key == pos ? vnew : vbase + (size_t)key * HD) + kVc * lane;
-            vcols_t v = {};
-            if (key < end) v = *reinterpret_cast<const vcols_t*>(row);
-#pragma unroll
-            for (int c = 0; c < kVc; ++c) vraw[j][c] = (float)v[c];
+        for (int j = 0; j < 4; ++j) {
+            const int vrow = first + 16 * wave + 4 * t + j;
+            vf[j] = *reinterpret_cast<const vcols_t*>(vbase + (size_t)(vrow < max_seq ? vrow : max_seq - 1) * HD +
+                                                      VC * col);
         }
     };
     load(start);
+    half8_t qraw[kSteps], kraw[kSteps];
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) qraw[st] = *reinterpret_cast<const half8_t*>(qh + 32 * st + 8 * t);
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) kraw[st] = *reinterpret_cast<const half8_t*>(knew + 32 * st + 8 * t);
+    const vcols_t vrow_new = *reinterpret_cast<const vcols_t*>(vnew + VC * col);
 
-    // RoPE of this lane's 8 columns of the query heads and of the new key.
-    float cs[8], sn[8];
+    if (pos64 < 0 || pos64 >= max_seq || start > pos64) return;
+    const int pos = (int)pos64;
+    const int end = start + chunk < pos + 1 ? start + chunk : pos + 1;
+
+    // RoPE of this lane's columns 32 st + 8 t .. + 7 of its head, and of the
+    // new key; exp(x / sqrt(HD) - max) = exp2((x - max) log2(e) / sqrt(HD)).
+    const float scale = kQScale * 1.4426950408889634f / sqrtf((float)HD);
+    half8_t qhi[kSteps], qlo[kSteps], kn[kSteps];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        cs[e] = cosp[(size_t)pos * HD + d0 + e];
-        sn[e] = sinp[(size_t)pos * HD + d0 + e];
+    for (int st = 0; st < kSteps; ++st) {
+        const bool low = st < kSteps / 2;
+        const int other = low ? st + kSteps / 2 : st - kSteps / 2;
+        const floatx4* c = reinterpret_cast<const floatx4*>(cosp + (size_t)pos * HD + 32 * st + 8 * t);
+        const floatx4* s = reinterpret_cast<const floatx4*>(sinp + (size_t)pos * HD + 32 * st + 8 * t);
+        const floatx4 cs[2] = {c[0], c[1]}, sn[2] = {s[0], s[1]};
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float cc = cs[e / 4][e % 4], ss = low ? -sn[e / 4][e % 4] : sn[e / 4][e % 4];
+            x[e] = ((float)qraw[st][e] * cc + (float)qraw[other][e] * ss) * scale;
+            kn[st][e] = (half_t)((float)kraw[st][e] * cc + (float)kraw[other][e] * ss);
+        }
+        split16(x, qhi[st], qlo[st]);
     }
-    float q[G][8];
+    if (end == pos + 1 && blockIdx.z == 0 && wave == 0) {   // the caches' new row
+        if (col == 0) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-        const half_t* qh = qkv + (size_t)(g * groups + h0 + (h < heads ? h : 0)) * HD;
-        const half8_t a = *reinterpret_cast<const half8_t*>(qh + d0);
-        const half8_t b = *reinterpret_cast<const half8_t*>(qh + dp);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) q[h][e] = rope((float)a[e], (float)b[e], cs[e], sn[e], low);
-    }
-    half8_t kn;
-    {
-        const half8_t a = *reinterpret_cast<const half8_t*>(knew + d0);
-        const half8_t b = *reinterpret_cast<const half8_t*>(knew + dp);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) kn[e] = (half_t)rope((float)a[e], (float)b[e], cs[e], sn[e], low);
-    }
-    if (end == pos + 1 && blockIdx.z == 0 && threadIdx.x < kLpk) {   // the cache's new row
-        *reinterpret_cast<half8_t*>(kbase + (size_t)pos * HD + d0) = kn;
-        *reinterpret_cast<half8_t*>(vbase + (size_t)pos * HD + d0) = *reinterpret_cast<const half8_t*>(vnew + d0);
+            for (int st = 0; st < kSteps; ++st)
+                *reinterpret_cast<half8_t*>(kbase + (size_t)pos * HD + 32 * st + 8 * t) = kn[st];
+        }
+        if (t == 0) *reinterpret_cast<vcols_t*>(vbase + (size_t)pos * HD + VC * col) = vrow_new;
     }
 
-    // exp(x / sqrt(HD) - max) = exp2(x c - max c)
-    const float c2 = 1.4426950408889634f / sqrtf((float)HD);
-    float m[G], l[G], o[G][kVc];
+    float m = -INFINITY, l = 0.0f;   // of head `col`; l: this lane's positions only
+    floatx4 acc[VC];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-        m[h] = -INFINITY;
-        l[h] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < kVc; ++c) o[h][c] = 0.0f;
-    }
-
+    for (int v = 0; v < VC; ++v) acc[v] = floatx4{0.f, 0.f, 0.f, 0.f};
     for (int first = start; first < end; first += kKeys) {
         if (first != start) load(first);
-        float s[kPass][G];
+        const int k0 = first + 16 * wave;
+        // The new position's row comes from the projection (the cache's may
+        // not be written yet), rows past it count as zeros.
+        if (k0 + col == pos) {
 #pragma unroll
-        for (int i = 0; i < kPass; ++i) {
-            const int key = first + 16 * wave + i * kRows + kr;
-            const half8_t kv = key == pos ? kn : kraw[i];
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                float a = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) a = fmaf((float)kv[e], q[h][e], a);
-                a = group_sum<kLpk>(a) * c2;
-                s[i][h] = key < end ? a : -INFINITY;
-            }
+            for (int st = 0; st < kSteps; ++st) kf[st] = kn[st];
         }
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
-            float mx = s[0][h];
-#pragma unroll
-            for (int i = 1; i < kPass; ++i) mx = fmaxf(mx, s[i][h]);
-#pragma unroll
-            for (int w = kLpk; w < 64; w *= 2) mx = fmaxf(mx, __shfl_xor(mx, w));
-            const float mn = fmaxf(m[h], mx);
-            const float ref = mn == -INFINITY ? 0.0f : mn;   // nothing yet: every exponential is 0
-            const float alpha = __builtin_amdgcn_exp2f(m[h] - ref);
-            float sum = 0.0f;
-#pragma unroll
-            for (int i = 0; i < kPass; ++i) {
-                const float p = __builtin_amdgcn_exp2f(s[i][h] - ref);
-                if (sub == 0) p_lds[wave][i * kRows + kr][h] = p;
-                sum += p;
-            }
-#pragma unroll
-            for (int w = kLpk; w < 64; w *= 2) sum += __shfl_xor(sum, w);
-            m[h] = mn;
-            l[h] = l[h] * alpha + sum;
-#pragma unroll
-            for (int c = 0; c < kVc; ++c) o[h][c] *= alpha;
+        for (int j = 0; j < 4; ++j) {
+            const int key = k0 + 4 * t + j;
+            if (key >= pos) vf[j] = key == pos ? vrow_new : vcols_t{};
         }
-        __builtin_amdgcn_wave_barrier();   // p_lds[wave] is written and read by this wave only, in order
+        floatx4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
+        for (int st = 0; st < kSteps; ++st) {
+            s = mfma16x16x32(kf[st], qhi[st], s);
+            s = mfma16x16x32(kf[st], qlo[st], s);
+        }
+        float mx = -INFINITY;
 #pragma unroll
-            for (int h = 0; h < G; ++h) {
-                const float p = p_lds[wave][j][h];
+        for (int r = 0; r < 4; ++r) {
+            if (k0 + 4 * t + r >= end) s[r] = -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mn = fmaxf(m, mx);
+        const float ref = mn == -INFINITY ? 0.0f : mn / kQScale;   // nothing yet: every exponential is 0
+        const float alpha = __builtin_amdgcn_exp2f(m / kQScale - ref);
+        m = mn;
+        float p[4];
+        l *= alpha;
 #pragma unroll
-                for (int c = 0; c < kVc; ++c) o[h][c] = fmaf(p, vraw[j][c], o[h][c]);
-            }
-        __builtin_amdgcn_wave_barrier();
+        for (int r = 0; r < 4; ++r) {
+            p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], 1.0f / kQScale, kPExp - ref));
+            l += p[r];
+        }
+        half4_t phi, plo;
+        split16(p, phi, plo);
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+            const half4_t a = {vf[0][v], vf[1][v], vf[2][v], vf[3][v]};
+            acc[v] *= alpha;
+            acc[v] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, phi, acc[v], 0, 0, 0);
+            acc[v] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, plo, acc[v], 0, 0, 0);
+        }
     }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
 
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-        if (lane == 0) {
-            m_lds[wave][h] = m[h];
-            l_lds[wave][h] = l[h];
+    // This lane: rows 4 t + r of each product, i.e. columns VC (4 t + r) + v of head `col`.
+    if (col < heads) {
+        if (t == 0) {
+            m_lds[wave][col] = m;
+            l_lds[wave][col] = l;
         }
 #pragma unroll
-        for (int c = 0; c < kVc; ++c) o_lds[wave][h][kVc * lane + c] = o[h][c];
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int v = 0; v < VC; v += 4)
+                *reinterpret_cast<floatx4*>(&o_lds[wave][col][VC * (4 * t + r) + v]) =
+                    floatx4{acc[v][r], acc[v + 1][r], acc[v + 2][r], acc[v + 3][r]};
     }
     __syncthreads();
     // part: [split][head][HD + 2]: HD sums, the maximum, the sum of exponentials
@@ -213,14 +213,14 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
         float sum = 0.0f, ls = 0.0f;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const float a = __builtin_amdgcn_exp2f(m_lds[w][h] - ref);
+            const float a = __builtin_amdgcn_exp2f((m_lds[w][h] - ref) / kQScale);
             sum = fmaf(a, o_lds[w][h][d], sum);
             ls = fmaf(a, l_lds[w][h], ls);
         }
         float* dst = part + ((size_t)split * nh + g * groups + h0 + h) * (HD + 2);
         dst[d] = sum;
         if (d == 0) {
-            dst[HD] = mx;
+            dst[HD] = mx / kQScale;
             dst[HD + 1] = ls;
         }
     }
@@ -266,34 +266,23 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
         out[(size_t)head * HD + d] = (half_t)((o_lds[0][d] + o_lds[1][d] + o_lds[2][d] + o_lds[3][d]) / l);
 }
 
-// Ranges of a cache of max_seq positions: 64 positions each, at most 64
-// ranges (longer caches take a multiple of 64 positions per range).
+// Ranges of a cache of max_seq positions: one inner pass each, at most 64
+// ranges (longer caches take a multiple of that per range).
 constexpr int kMaxRanges = 64;
 int chunk_for(int64_t max_seq) { return (int)(kKeys * ((max_seq + kMaxRanges * kKeys - 1) / (kMaxRanges * kKeys))); }
 
-template <int HD, int G>
+template <int HD>
 hipError_t launch(const DecodeAttnArgs& a, hipStream_t stream) {
     const int groups = a.nh / a.kvh, chunk = chunk_for(a.max_seq);
     const int splits = (a.max_seq + chunk - 1) / chunk;
-    hipLaunchKernelGGL((awq_decode_attn_kernel<HD, G>), dim3(splits, a.kvh, (groups + G - 1) / G), dim3(kThreads), 0,
-                       stream, a.qkv, a.k_cache, a.v_cache, a.cos, a.sin, a.pos, a.part, a.nh, a.kvh, groups,
-                       a.max_seq, chunk);
+    hipLaunchKernelGGL((awq_decode_attn_kernel<HD>), dim3(splits, a.kvh, (groups + kHeads - 1) / kHeads),
+                       dim3(kThreads), 0, stream, a.qkv, a.k_cache, a.v_cache, a.cos, a.sin, a.pos, a.part, a.nh,
+                       a.kvh, groups, a.max_seq, chunk);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((awq_decode_combine_kernel<HD>), dim3(a.nh), dim3(4 * HD), 0, stream, a.part, a.pos, a.out,
                        a.nh, a.max_seq, chunk);
     return hipGetLastError();
-}
-
-// Query heads per workgroup: all of a KV head's up to 8 (K and V are then
-// read once), the smallest instance that holds them.
-template <int HD>
-hipError_t launch_hd(const DecodeAttnArgs& a, hipStream_t stream) {
-    const int groups = a.nh / a.kvh;
-    if (groups == 1) return launch<HD, 1>(a, stream);
-    if (groups == 2) return launch<HD, 2>(a, stream);
-    if (groups <= 4) return launch<HD, 4>(a, stream);
-    return launch<HD, 8>(a, stream);
 }
 
 }  // namespace
@@ -304,7 +293,7 @@ size_t decode_attn_workspace(int max_seq, int nh, int hd) {
 }
 
 hipError_t launch_decode_attn(const DecodeAttnArgs& a, int hd, hipStream_t stream) {
-    return hd == 64 ? launch_hd<64>(a, stream) : launch_hd<128>(a, stream);
+    return hd == 64 ? launch<64>(a, stream) : launch<128>(a, stream);
 }
 
 }  // namespace awq

@@ -52,12 +52,13 @@ def _close(y, ref, what):
 
 @pytest.mark.parametrize("nh,kvh,hd,max_seq,positions", [
     (28, 4, 128, 1152, (0, 1, 15, 16, 63, 64, 65, 1023, 1151)),
-    (28, 4, 128, 5000, (127, 128, 4095, 4999)),        # ranges of 128 positions
+    (28, 4, 128, 5000, (127, 128, 4095, 4999)),
+    (4, 2, 64, 20000, (383, 384, 511, 512, 19999)),    # ranges of several passes
     (4, 2, 64, 64, (0, 7, 63)),
     (6, 2, 64, 130, (128, 129)),
-    (12, 1, 64, 100, (99,)),                           # more query heads than one workgroup takes
+    (18, 1, 64, 300, (99, 271)),                       # more query heads than one workgroup takes
     (3, 3, 128, 1, (0,)),
-    (18, 2, 128, 70, (64, 69)),
+    (34, 2, 128, 70, (64, 69)),
 ])
 def test_attention_decode(gpu, nh, kvh, hd, max_seq, positions):
     g = torch.Generator().manual_seed(max_seq)
