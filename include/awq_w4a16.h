@@ -302,6 +302,24 @@ int awq_w4a16_gemm_epilogue(const void* x, const int32_t* qweight, const int32_t
                             int64_t M, int64_t N, int64_t K, int32_t group_size, void* workspace,
                             size_t workspace_bytes, const awq_w4a16_plan* plan, void* stream);
 
+/* One decode row's projection with the step before it fused into the kernel's
+ * prologue (M = 1, the AUTO plan): out[1, N] = row @ W, then bias / residual as
+ * in awq_w4a16_gemm_epilogue, where
+ *   AWQ_INPUT_RMSNORM   row = fp16(x * rsqrt(mean(x^2) + eps) * norm_w), x and
+ *                       norm_w fp16 [K] (model/qwen2.py:15-22);
+ *   AWQ_INPUT_SILU_MUL  row = fp16(silu(x[k]) * x[K + k]), x fp16 [2 K], the fused
+ *                       gate||up projection (kernels/silu_mul.py:17-39); norm_w
+ *                       and eps are not read.
+ * awq_w4a16_decode_served: 1 where the shape's AUTO plan has such a prologue, 0
+ * where the call returns AWQ_ERR_PATH and the caller makes the row itself. */
+#define AWQ_INPUT_RMSNORM 1
+#define AWQ_INPUT_SILU_MUL 2
+int awq_w4a16_decode_served(int64_t N, int64_t K, int32_t group_size, int32_t input);
+int awq_w4a16_gemm_decode(int32_t input, const void* x, const void* norm_w, float eps, const int32_t* qweight,
+                          const int32_t* qzeros, const void* scales, const void* bias, const void* residual,
+                          void* out, int64_t N, int64_t K, int32_t group_size, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* out[m, i] = fp16(silu(g) * u), g = gate_up[m, i], u = gate_up[m, I + i], in
  * fp32 with one rounding: the reference's silu_mul (kernels/silu_mul.py:17-39)
  * over the fused gate||up projection read in place, replacing its two

@@ -781,9 +781,13 @@ int check_pointers(const void* x, const void* qweight, const void* qzeros, const
 
 int run_plan(const void* x, const int32_t* qweight, const int32_t* qzeros, const void* scales,
              void* out, int64_t M, int64_t N, int64_t K, void* workspace, const awq_w4a16_plan& p,
-             void* stream, const void* bias = nullptr, const void* residual = nullptr) {
+             void* stream, const void* bias = nullptr, const void* residual = nullptr, int input = kInputX,
+             const void* norm_w = nullptr, float norm_eps = 0.0f) {
     if (M == 0) return AWQ_OK;
     GemmArgs a;
+    a.input = input;
+    a.norm_w = static_cast<const half_t*>(norm_w);
+    a.norm_eps = norm_eps;
     a.bias = static_cast<const half_t*>(bias);
     a.residual = static_cast<const half_t*>(residual);
     a.x = static_cast<const half_t*>(x);
@@ -841,6 +845,17 @@ int run_plan(const void* x, const int32_t* qweight, const int32_t* qzeros, const
         e = launch_tile(a, cfg, static_cast<uint32_t*>(workspace), s);
     }
     return e == hipSuccess ? AWQ_OK : AWQ_ERR_LAUNCH;
+}
+
+// The AUTO plan of one decode row whose prologue can make it: the column GEMVs
+// with two chunk buffers, and for the norm a row that its threads hold.
+int decode_plan(int64_t N, int64_t K, int32_t group_size, int32_t input, awq_w4a16_plan* p) {
+    if (input != AWQ_INPUT_RMSNORM && input != AWQ_INPUT_SILU_MUL) return AWQ_ERR_PATH;
+    const int st = awq_w4a16_plan_for(1, N, K, group_size, AWQ_PATH_AUTO, p);
+    if (st != AWQ_OK) return st;
+    if (p->path != AWQ_PATH_GEMV || p->variant != 5 || p->depth != 2) return AWQ_ERR_PATH;
+    if (input == AWQ_INPUT_RMSNORM && K > gemv_norm_max_k(p->k_waves)) return AWQ_ERR_PATH;
+    return AWQ_OK;
 }
 
 // ---- the allocation-free entry point (awq_w4a16_gemm_noalloc) ---------------
@@ -1129,6 +1144,31 @@ int awq_w4a16_gemm_epilogue(const void* x, const int32_t* qweight, const int32_t
         awq_w4a16_plan_for(M, N, K, group_size, AWQ_PATH_AUTO, &p);
     }
     return run_plan(x, qweight, qzeros, scales, out, M, N, K, workspace, p, stream, bias, residual);
+}
+
+int awq_w4a16_decode_served(int64_t N, int64_t K, int32_t group_size, int32_t input) {
+    awq_w4a16_plan p;
+    return decode_plan(N, K, group_size, input, &p) == AWQ_OK ? 1 : 0;
+}
+
+int awq_w4a16_gemm_decode(int32_t input, const void* x, const void* norm_w, float eps, const int32_t* qweight,
+                          const int32_t* qzeros, const void* scales, const void* bias, const void* residual,
+                          void* out, int64_t N, int64_t K, int32_t group_size, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+    awq_w4a16_plan p;
+    int st = decode_plan(N, K, group_size, input, &p);
+    if (st != AWQ_OK) return st;
+    st = check_pointers(x, qweight, qzeros, scales, out, 1);
+    if (st != AWQ_OK) return st;
+    if (input == AWQ_INPUT_RMSNORM && !norm_w) return AWQ_ERR_NULL_POINTER;
+    if (input == AWQ_INPUT_RMSNORM && !aligned(norm_w, 16)) return AWQ_ERR_MISALIGNED;
+    if ((bias && !aligned(bias, 2)) || (residual && !aligned(residual, 2))) return AWQ_ERR_MISALIGNED;
+    if (p.workspace_bytes > 0) {
+        if (!workspace || workspace_bytes < p.workspace_bytes) return AWQ_ERR_WORKSPACE;
+        if (!aligned(workspace, 16)) return AWQ_ERR_MISALIGNED;
+    }
+    return run_plan(x, qweight, qzeros, scales, out, 1, N, K, workspace, p, stream, bias, residual,
+                    input == AWQ_INPUT_RMSNORM ? kInputNorm : kInputSiluMul, norm_w, eps);
 }
 
 int awq_w4a16_gemm_noalloc(const void* x, const int32_t* qweight, const int32_t* qzeros, const void* scales,

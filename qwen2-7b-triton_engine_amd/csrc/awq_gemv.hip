@@ -238,9 +238,18 @@ __global__ __launch_bounds__(512) void awq_gemv_stream_kernel(GemmArgs a, int ch
 // s(b + z) * sum_x for the M live rows.  At the end the waves are added
 // through LDS and each output's partial is stored (split_k == 1) or goes
 // through the fixed-point finish.  Needs N % 32 == 0 (whole quads).
+//
+// IN (M == 1): the row of x is made in the prologue, while the first weight
+// chunks are in flight, from what the decode step has at hand -- kInputNorm
+// takes the RMSNorm of the row (every workgroup sums the whole row's squares,
+// 7 KB from L2, and scales its own K range), kInputSiluMul takes SiLU(gate) *
+// up of its K range.  A launch in a replayed graph costs 2.1 us however small;
+// measured in graphs over 28 layers' weights, us, fused / two launches: norm
+// + 3584 x 4608 6.3 / 7.7, norm + 3584 x 37888 17.4 / 18.8, SiLU * up + 18944 x
+// 3584 11.4 / 13.5; a decoder layer 53.7 / 57.7.
 constexpr int kQuadItemsPerThread = 4;  // prologue loads per thread (consts and x each)
 
-template <int MR, int D, bool NT, int CW, bool RED = false>
+template <int MR, int D, bool NT, int CW, bool RED = false, int IN = kInputX>
 __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int split_k, unsigned long long* fix) {
     extern __shared__ __align__(16) uint32_t lds[];
     const int lane = threadIdx.x & 63;
@@ -255,6 +264,7 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
     constexpr int NR = MR > 4 ? 4 : MR;
     constexpr int XI = MR > 8 ? 16 : (MR > 4 ? 8 : kQuadItemsPerThread);  // x prologue loads per thread
     static_assert(MR <= 8 || RED, "16 rows of x take the reduce-launch finish");
+    static_assert(IN == kInputX || MR == 1, "a made input is one row");
     const int pn = a.N >> 3;
     const int n_strips = (pn + SP - 1) / SP;
     // Work item w = (split, strip), strip fastest, numbered in XCD order:
@@ -280,7 +290,8 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.qweight, (uint32_t)((size_t)a.K * pn * 4));
     const __amdgpu_buffer_rsrc_t rz = make_rsrc(a.qzeros, (uint32_t)((size_t)groups * pn * 4));
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.scales, (uint32_t)((size_t)groups * a.N * 2));
-    const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, (uint32_t)((size_t)a.M * a.K * 2));
+    const __amdgpu_buffer_rsrc_t rx =
+        make_rsrc(a.x, (uint32_t)((size_t)a.M * a.K * (IN == kInputSiluMul ? 4 : 2)));
     const uint32_t row_bytes = (uint32_t)pn * 4u;
     const uint32_t voff_w = (uint32_t)(4 * rq) * row_bytes + (uint32_t)jl * 4u;
 
@@ -311,6 +322,23 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
         const int m = xi / max(nc * 4, 1);
         const uint32_t xoff = (uint32_t)(((size_t)m * a.K + (size_t)c0 * 32 + 8 * (xi % max(nc * 4, 1))) * 2);
         xv[i] = buf_load_u4(rx, m < MR ? xoff : 0x80000000u, 0u);
+    }
+    // The made inputs' other operand (the norm's weight or up), and for the
+    // norm the whole row (pieces past it read zeros).
+    u32x4 xw[IN == kInputX ? 1 : XI], row[IN == kInputNorm ? kQuadItemsPerThread : 1];
+    if constexpr (IN != kInputX) {
+        const __amdgpu_buffer_rsrc_t rn = IN == kInputNorm ? make_rsrc(a.norm_w, (uint32_t)a.K * 2u) : rx;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int xi = (int)threadIdx.x + i * nt;
+            const uint32_t off = (uint32_t)(c0 * 32 + 8 * xi + (IN == kInputSiluMul ? a.K : 0)) * 2u;
+            xw[i] = buf_load_u4(rn, xi < nc * 4 ? off : 0x80000000u, 0u);
+        }
+    }
+    if constexpr (IN == kInputNorm) {
+#pragma unroll
+        for (int i = 0; i < kQuadItemsPerThread; ++i)
+            row[i] = buf_load_u4(rx, (uint32_t)((int)threadIdx.x + i * nt) * 16u, 0u);
     }
 
     typedef uint32_t cwv_t __attribute__((ext_vector_type(CW < 2 ? 2 : CW)));
@@ -375,6 +403,44 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
                 const int col = 8 * (j % CW) + c;  // column of the lane: pair index col / 2
                 lc[(g * (4 * CW) + col / 2) * 16 + j / CW] = v;
             }
+        }
+    }
+    if constexpr (IN == kInputNorm) {
+        __shared__ float squares[8];   // per wave
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < kQuadItemsPerThread; ++i) {
+            const half8_t v = __builtin_bit_cast(half8_t, row[i]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)v[e], (float)v[e], s);
+        }
+#pragma unroll
+        for (int w = 1; w < 64; w *= 2) s += __shfl_xor(s, w);
+        if (lane == 0) squares[wave] = s;
+        __syncthreads();
+        s = 0.f;
+        for (int w = 0; w < nw; ++w) s += squares[w];
+        const float r = 1.0f / sqrtf(s / (float)a.K + a.norm_eps);
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            half8_t v = __builtin_bit_cast(half8_t, xv[i]);
+            const half8_t w = __builtin_bit_cast(half8_t, xw[i]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = (half_t)((float)v[e] * r * (float)w[e]);
+            xv[i] = __builtin_bit_cast(u32x4, v);
+        }
+    } else if constexpr (IN == kInputSiluMul) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            if ((int)threadIdx.x + i * nt >= nc * 4) continue;
+            half8_t v = __builtin_bit_cast(half8_t, xv[i]);
+            const half8_t u = __builtin_bit_cast(half8_t, xw[i]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float x = (float)v[e];
+                v[e] = (half_t)(x / (1.0f + expf(-x)) * (float)u[e]);
+            }
+            xv[i] = __builtin_bit_cast(u32x4, v);
         }
     }
 #pragma unroll
@@ -540,7 +606,9 @@ static hipError_t gemv_stream_launch(const GemmArgs& a, const GemvConfig& cfg, u
     return hipGetLastError();
 }
 
-template <int MR, int D, int CW, bool RED = false>
+int gemv_norm_max_k(int k_waves) { return kQuadItemsPerThread * 64 * k_waves * 8; }
+
+template <int MR, int D, int CW, bool RED = false, int IN = kInputX>
 static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uint32_t* counters,
                                    hipStream_t stream) {
     unsigned long long* fix = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(counters) + kCounterBytes);
@@ -551,16 +619,30 @@ static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uin
     // faster with them at M = 1 - 16, the 100 - 500-row ranges of 18 - 36
     // splits up to 3 % slower.
     if (cfg.split_k <= kNonTemporalMaxSplit)
-        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, true, CW, RED>), grid, block, lds, stream, a, cfg.split_k, fix);
+        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, true, CW, RED, IN>), grid, block, lds, stream, a, cfg.split_k, fix);
     else
-        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, false, CW, RED>), grid, block, lds, stream, a, cfg.split_k, fix);
+        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, false, CW, RED, IN>), grid, block, lds, stream, a, cfg.split_k, fix);
     const hipError_t e = hipGetLastError();
     if (!RED || e != hipSuccess || cfg.split_k <= 1) return e;
     return splitk_reduce_launch(a, cfg.split_k, stream);
 }
 
+template <int IN>
+static hipError_t gemv_quad_input_dispatch(const GemmArgs& a, const GemvConfig& cfg, uint32_t* counters,
+                                           hipStream_t stream) {
+    if (a.M != 1 || cfg.depth != 2) return hipErrorInvalidValue;
+    switch (cfg.cw) {
+        case 1: return gemv_quad_launch<1, 2, 1, false, IN>(a, cfg, counters, stream);
+        case 2: return gemv_quad_launch<1, 2, 2, false, IN>(a, cfg, counters, stream);
+        case 4: return gemv_quad_launch<1, 2, 4, false, IN>(a, cfg, counters, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 static hipError_t gemv_quad_dispatch(const GemmArgs& a, const GemvConfig& cfg, uint32_t* counters,
                                      hipStream_t stream) {
+    if (a.input == kInputNorm) return gemv_quad_input_dispatch<kInputNorm>(a, cfg, counters, stream);
+    if (a.input == kInputSiluMul) return gemv_quad_input_dispatch<kInputSiluMul>(a, cfg, counters, stream);
     if (cfg.cw == 1) {
         switch (gemv_quad_mr(a.M) * 10 + cfg.depth) {
             case 12: return gemv_quad_launch<1, 2, 1>(a, cfg, counters, stream);

@@ -20,7 +20,15 @@ struct GemmArgs {
     int M, N, K;
     const half_t* bias = nullptr;      // [N] added to every row (epilogue), or null
     const half_t* residual = nullptr;  // [M, N] added after the bias (epilogue), or null; may alias out
+    // How the decode GEMV's prologue makes its row of x (kInput*; M == 1,
+    // launch_gemv variant 5 with depth 2 only; every other launch takes kInputX).
+    int input = 0;
+    const half_t* norm_w = nullptr;    // kInputNorm: [K]
+    float norm_eps = 0.0f;
 };
+// x is the row; x is normalised on the way: fp16(x * rsqrt(mean(x^2) + eps) *
+// w); x is gate||up [2 K] and the row is fp16(silu(gate) * up).
+constexpr int kInputX = 0, kInputNorm = 1, kInputSiluMul = 2;
 
 struct SkinnyConfig {
     int m_blocks;            // 16-row MFMA blocks of x: 1, 2 or 4
@@ -132,6 +140,8 @@ int64_t gemv_strips(int N);
 int64_t gemv_strips_cw(int N, int cw);
 size_t gemv_quad_lds_bytes(int M, int K, int split_k, int k_waves, int cw);
 int64_t gemv_quad_max_groups(int K, int split_k);
+// Longest row kInputNorm serves: four 16-byte pieces of it per thread.
+int gemv_norm_max_k(int k_waves);
 bool gemv_quad_fits(int M, int K, int split_k, int k_waves, int cw);
 
 // Stream path (M <= 16, N % 32 == 0, split_k <= K / 128).  layout:

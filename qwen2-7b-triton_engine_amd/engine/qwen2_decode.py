@@ -31,7 +31,8 @@ import time
 import torch
 
 from kernels.attention import attention_decode, attention_prefill, attention_served
-from kernels.awq_gemm import awq_gemm_forward, awq_gemm_forward_ex
+from kernels._native import INPUT_RMSNORM, INPUT_SILU_MUL
+from kernels.awq_gemm import awq_gemm_decode, awq_gemm_forward, awq_gemm_forward_ex, decode_linear_served
 from kernels.lm_head import lm_head_forward
 from kernels.rmsnorm import MAX_H, rmsnorm
 from kernels.silu_mul import silu_mul_gate_up
@@ -174,15 +175,24 @@ class Qwen2AwqDecoder:
 
     # ---- one decoder layer over positions `pos` (device int64 [S]) -------------
     def _layer(self, li: int, h: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
-        s = self.s
         p = self.layers[li]
-        x = _rmsnorm(h, p["ln1"], s.rms_norm_eps)
-        qkv = self.linear(x, p["qkv"], bias=p["qkv_bias"])
+        qkv = self._normed_linear(h, p["ln1"], p["qkv"], bias=p["qkv_bias"])
         att = self._attention(li, qkv, pos, causal)
         h = self.linear(att, p["o"], residual=h)
-        x = _rmsnorm(h, p["ln2"], s.rms_norm_eps)
-        inter = silu_mul_gate_up(self.linear(x, p["gate_up"]))
-        return self.linear(inter, p["down"], residual=h)
+        gate_up = self._normed_linear(h, p["ln2"], p["gate_up"])
+        if self._one_row(gate_up, p["down"], INPUT_SILU_MUL):
+            return awq_gemm_decode(INPUT_SILU_MUL, gate_up, *p["down"], residual=h)
+        return self.linear(silu_mul_gate_up(gate_up), p["down"], residual=h)
+
+    def _one_row(self, x: torch.Tensor, op, kind: int) -> bool:
+        """Whether this is a decode row that the projection `op` makes its input of."""
+        return x.shape[0] == 1 and decode_linear_served(op[2].shape[1], op[0].shape[0], kind)
+
+    def _normed_linear(self, h: torch.Tensor, w: torch.Tensor, op, bias: torch.Tensor | None = None) -> torch.Tensor:
+        """The projection `op` of RMSNorm(h)."""
+        if w.dtype == torch.float16 and h.dtype == torch.float16 and self._one_row(h, op, INPUT_RMSNORM):
+            return awq_gemm_decode(INPUT_RMSNORM, h, *op, norm_w=w, eps=self.s.rms_norm_eps, bias=bias)
+        return self.linear(_rmsnorm(h, w, self.s.rms_norm_eps), op, bias=bias)
 
     def _attention(self, li: int, qkv: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         """Attention output fp16 [S, heads * head_dim] of the positions `pos`,

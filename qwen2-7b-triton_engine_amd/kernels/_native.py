@@ -27,6 +27,9 @@ AWQ_ERR_CAPTURE = -10
 NOALLOC_SCRATCH_BYTES = 32 << 20
 SLOT_BYTES = 2 << 20   # fixed-point slot region of a workspace (AWQ_W4A16_SLOT_BYTES)
 
+INPUT_RMSNORM = 1
+INPUT_SILU_MUL = 2
+
 PATH_AUTO = 0
 PATH_SKINNY = 1
 PATH_TILE = 2
@@ -91,6 +94,9 @@ SIGNATURES = {
     "awq_w4a16_gemm_epilogue": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I32, _VP,
                                                ctypes.c_size_t, ctypes.POINTER(Plan), _VP]),
     "awq_silu_mul": (ctypes.c_int, [_VP, _VP, _I64, _I64, _VP]),
+    "awq_w4a16_decode_served": (ctypes.c_int, [_I64, _I64, _I32, _I32]),
+    "awq_w4a16_gemm_decode": (ctypes.c_int, [_I32, _VP, _VP, ctypes.c_float, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64,
+                                             _I32, _VP, ctypes.c_size_t, _VP]),
     "awq_fp16_rmsnorm": (ctypes.c_int, [_VP, _VP, _VP, _I64, _I64, ctypes.c_float, _VP]),
     "awq_fp16_attention_decode_workspace": (ctypes.c_size_t, [_I64, _I64, _I64, _I64]),
     "awq_fp16_attention_decode": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I64, _I64, _VP,

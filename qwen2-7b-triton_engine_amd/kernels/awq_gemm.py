@@ -43,7 +43,7 @@ import torch
 
 from . import _native
 
-__all__ = ["awq_gemm_forward", "awq_gemm_forward_ex", "_dequant_to_fp16", "plan"]
+__all__ = ["awq_gemm_forward", "awq_gemm_forward_ex", "awq_gemm_decode", "decode_linear_served", "_dequant_to_fp16", "plan"]
 
 
 _F16, _I32 = torch.float16, torch.int32
@@ -268,6 +268,47 @@ def awq_gemm_forward_ex(x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Te
     _launch(x_flat, qweight, qzeros, scales, out, M, N, K, group_size, dev, path=path, plan_obj=plan_obj,
             bias=bias, residual=residual)
     return out.view(*in_shape[:-1], N)
+
+
+def decode_linear_served(n: int, k: int, input: int, group_size: int = 128) -> bool:
+    """Whether ``awq_gemm_decode`` serves ``[1, k] x [k, n]`` with this input."""
+    return bool(_native.lib().awq_w4a16_decode_served(n, k, group_size, input))
+
+
+def awq_gemm_decode(input: int, x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
+                    norm_w: torch.Tensor | None = None, eps: float = 0.0, bias: torch.Tensor | None = None,
+                    residual: torch.Tensor | None = None, group_size: int = 128) -> torch.Tensor:
+    """One decode row's projection ``[1, N]`` with the step before it in the
+    kernel's prologue: ``input`` ``_native.INPUT_RMSNORM`` (``x [1, K]``, normalised
+    with ``norm_w`` and ``eps``) or ``_native.INPUT_SILU_MUL`` (``x [1, 2K]``, gate||up).
+    Shapes without such a kernel (``decode_linear_served``) raise ``ValueError``."""
+    K, N = qweight.shape[0], scales.shape[1]
+    width = 2 * K if input == _native.INPUT_SILU_MUL else K
+    if x.shape != (1, width):
+        raise ValueError(f"x must be [1, {width}], got {tuple(x.shape)}")
+    _check_operands(x[:, :K], qweight, qzeros, scales, group_size)
+    dev = _check_device(x, qweight, qzeros, scales)
+    for t, what, n in ((norm_w, "norm_w", K), (bias, "bias", N), (residual, "residual", N)):
+        if t is not None and (t.dtype != torch.float16 or t.numel() != n or t.device != dev):
+            raise ValueError(f"{what} must be an fp16 tensor of {n} values on {dev}")
+    if (norm_w is None) == (input == _native.INPUT_RMSNORM):
+        raise ValueError("norm_w goes with the RMSNorm input")
+    if not decode_linear_served(N, K, input, group_size):
+        raise ValueError(f"no kernel makes input {input} for K={K}, N={N}")
+    flat = lambda t: None if t is None else t.contiguous()  # noqa: E731
+    x, qweight, qzeros, scales = _aligned16(x.contiguous()), flat(qweight), flat(qzeros), _aligned16(flat(scales))
+    norm_w, bias, residual = None if norm_w is None else _aligned16(flat(norm_w)), flat(bias), flat(residual)
+    out = torch.empty((1, N), dtype=torch.float16, device=dev)
+    p, _ = _plan_cached(1, N, K, group_size, _native.PATH_AUTO, dev)
+    ws = _workspace(dev, p.workspace_bytes) if p.workspace_bytes else None
+    with _OnDevice(dev):
+        st = _native.lib().awq_w4a16_gemm_decode(
+            input, x.data_ptr(), 0 if norm_w is None else norm_w.data_ptr(), eps, qweight.data_ptr(),
+            qzeros.data_ptr(), scales.data_ptr(), 0 if bias is None else bias.data_ptr(),
+            0 if residual is None else residual.data_ptr(), out.data_ptr(), N, K, group_size,
+            0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel() * 4, _stream_handle(dev))
+    _native.check(st, "awq_w4a16_gemm_decode")
+    return out
 
 
 def _dequant_to_fp16(qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
