@@ -11,15 +11,17 @@
 // enough workgroups to load it at once, each keeps a running softmax of its
 // range for all query heads of one KV head (so K and V are read once), and a
 // second launch weights the ranges' partial sums.  Measured on Qwen2-7B's
-// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 10.2 us
-// for the two at position 1100, 8.1 of it the first -- a form of it with the
-// scores, the softmax and P V on the vector unit, 16 lanes a key, took 15.3.
+// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 8.8 us for
+// the two at position 1100, where two empty launches take 4.2; 10.2 with eight
+// waves a workgroup (two per SIMD: the kernel is then bound by its own
+// instructions) and its loads behind the position's; 17 with the scores, the
+// softmax and P V on the vector unit, 16 lanes a key.
 #include "awq_kernels.h"
 
 namespace awq {
 namespace {
 
-constexpr int kThreads = 512;
+constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kHeads = 16;             // query heads of one workgroup: the columns of an MFMA
 constexpr int kKeys = 16 * kWaves;     // positions of one inner pass of a workgroup: 16 per wave
@@ -52,7 +54,11 @@ __device__ __forceinline__ void split16(float (&x)[N], V& hi, V& lo) {
 // cache past it are masked), so the chain is two memory latencies long: the
 // position, then the RoPE row it selects.  The waves' results meet once, at
 // the end.
-template <int HD>
+//
+// LONG: ranges of several passes.  Their workgroups past the position return
+// at once; a short range's go on (every position masked, nothing stored)
+// instead of keeping all loads behind the position's.
+template <int HD, bool LONG>
 __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
     const half_t* __restrict__ qkv, half_t* kc, half_t* vc, const float* __restrict__ cosp,
     const float* __restrict__ sinp, const int64_t* __restrict__ posp, float* __restrict__ part, int nh, int kvh,
@@ -92,6 +98,7 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
                                                       VC * col);
         }
     };
+    if (LONG && start > pos64) return;
     load(start);
     half8_t qraw[kSteps], kraw[kSteps];
 #pragma unroll
@@ -100,31 +107,38 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
     for (int st = 0; st < kSteps; ++st) kraw[st] = *reinterpret_cast<const half8_t*>(knew + 32 * st + 8 * t);
     const vcols_t vrow_new = *reinterpret_cast<const vcols_t*>(vnew + VC * col);
 
-    if (pos64 < 0 || pos64 >= max_seq || start > pos64) return;
-    const int pos = (int)pos64;
+    const bool valid = pos64 >= 0 && pos64 < max_seq;
+    const int pos = valid ? (int)pos64 : 0;
     const int end = start + chunk < pos + 1 ? start + chunk : pos + 1;
+    floatx4 cs[kSteps][2], sn[kSteps][2];
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            cs[st][e] = reinterpret_cast<const floatx4*>(cosp + (size_t)pos * HD + 32 * st + 8 * t)[e];
+            sn[st][e] = reinterpret_cast<const floatx4*>(sinp + (size_t)pos * HD + 32 * st + 8 * t)[e];
+        }
+    __builtin_amdgcn_sched_barrier(0);   // every load above is issued before the first is waited for
 
     // RoPE of this lane's columns 32 st + 8 t .. + 7 of its head, and of the
     // new key; exp(x / sqrt(HD) - max) = exp2((x - max) log2(e) / sqrt(HD)).
     const float scale = kQScale * 1.4426950408889634f / sqrtf((float)HD);
-    half8_t qhi[kSteps], qlo[kSteps], kn[kSteps];
+    const bool has_new = start <= pos && end == pos + 1;
+    half8_t qhi[kSteps], qlo[kSteps], kn[kSteps] = {};
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
         const bool low = st < kSteps / 2;
         const int other = low ? st + kSteps / 2 : st - kSteps / 2;
-        const floatx4* c = reinterpret_cast<const floatx4*>(cosp + (size_t)pos * HD + 32 * st + 8 * t);
-        const floatx4* s = reinterpret_cast<const floatx4*>(sinp + (size_t)pos * HD + 32 * st + 8 * t);
-        const floatx4 cs[2] = {c[0], c[1]}, sn[2] = {s[0], s[1]};
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float cc = cs[e / 4][e % 4], ss = low ? -sn[e / 4][e % 4] : sn[e / 4][e % 4];
+            const float cc = cs[st][e / 4][e % 4], ss = low ? -sn[st][e / 4][e % 4] : sn[st][e / 4][e % 4];
             x[e] = ((float)qraw[st][e] * cc + (float)qraw[other][e] * ss) * scale;
-            kn[st][e] = (half_t)((float)kraw[st][e] * cc + (float)kraw[other][e] * ss);
+            if (has_new) kn[st][e] = (half_t)((float)kraw[st][e] * cc + (float)kraw[other][e] * ss);
         }
         split16(x, qhi[st], qlo[st]);
     }
-    if (end == pos + 1 && blockIdx.z == 0 && wave == 0) {   // the caches' new row
+    if (valid && has_new && blockIdx.z == 0 && wave == 0) {   // the caches' new row
         if (col == 0) {
 #pragma unroll
             for (int st = 0; st < kSteps; ++st)
@@ -137,7 +151,7 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
     floatx4 acc[VC];
 #pragma unroll
     for (int v = 0; v < VC; ++v) acc[v] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int first = start; first < end; first += kKeys) {
+    for (int first = start; first == start || (LONG && first < end); first += kKeys) {
         if (first != start) load(first);
         const int k0 = first + 16 * wave;
         // The new position's row comes from the projection (the cache's may
@@ -202,6 +216,7 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
                 *reinterpret_cast<floatx4*>(&o_lds[wave][col][VC * (4 * t + r) + v]) =
                     floatx4{acc[v][r], acc[v + 1][r], acc[v + 2][r], acc[v + 3][r]};
     }
+    if (!valid || start > pos) return;   // the whole workgroup
     __syncthreads();
     // part: [split][head][HD + 2]: HD sums, the maximum, the sum of exponentials
     for (int i = threadIdx.x; i < heads * HD; i += kThreads) {
@@ -234,16 +249,26 @@ template <int HD>
 __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float* __restrict__ part,
                                                                     const int64_t* __restrict__ posp,
                                                                     half_t* __restrict__ out, int nh, int max_seq,
-                                                                    int chunk) {
+                                                                    int chunk, int ranges) {
     __shared__ float o_lds[4][HD];
     const int64_t pos = *posp;
-    if (pos < 0 || pos >= max_seq) return;
-    const int n = (int)(pos / chunk) + 1;
     const int head = blockIdx.x, d = threadIdx.x % HD, quarter = threadIdx.x / HD, lane = threadIdx.x & 63;
     const size_t step = (size_t)nh * (HD + 2);
     const float* base = part + (size_t)head * (HD + 2);
-    const float mine = lane < n ? base[lane * step + HD] : -INFINITY;
-    float l = lane < n ? base[lane * step + HD + 1] : 0.0f;
+    // Loaded before the position is known; what no range wrote this time is
+    // masked below.
+    const int lr = lane < ranges ? lane : 0;
+    float mine = base[lr * step + HD], l = base[lr * step + HD + 1];
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = base[(quarter + 4 * j < ranges ? quarter + 4 * j : 0) * step + d];
+    __builtin_amdgcn_sched_barrier(0);
+    if (pos < 0 || pos >= max_seq) return;
+    const int n = (int)pos / chunk + 1;
+    if (lane >= n) {
+        mine = -INFINITY;
+        l = 0.0f;
+    }
     float mx = mine;
 #pragma unroll
     for (int w = 1; w < 64; w *= 2) mx = fmaxf(mx, __shfl_xor(mx, w));
@@ -253,12 +278,15 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
     for (int w = 1; w < 64; w *= 2) l += __shfl_xor(l, w);
     float sum = 0.0f;
     for (int i0 = quarter; i0 < n; i0 += 32) {
-        float v[8];
+        if (i0 != quarter) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = i0 + 4 * j < n ? base[(i0 + 4 * j) * step + d] : 0.0f;
+            for (int j = 0; j < 8; ++j) v[j] = i0 + 4 * j < n ? base[(i0 + 4 * j) * step + d] : 0.0f;
+        }
 #pragma unroll
-        for (int j = 0; j < 8; ++j)   // lanes past n hold weight 0
-            sum = fmaf(__shfl(a, (i0 + 4 * j) & 63), v[j], sum);
+        for (int j = 0; j < 8; ++j) {
+            const float w = __shfl(a, (i0 + 4 * j) & 63);
+            sum = fmaf(w, i0 + 4 * j < n ? v[j] : 0.0f, sum);
+        }
     }
     o_lds[quarter][d] = sum;
     __syncthreads();
@@ -275,13 +303,14 @@ template <int HD>
 hipError_t launch(const DecodeAttnArgs& a, hipStream_t stream) {
     const int groups = a.nh / a.kvh, chunk = chunk_for(a.max_seq);
     const int splits = (a.max_seq + chunk - 1) / chunk;
-    hipLaunchKernelGGL((awq_decode_attn_kernel<HD>), dim3(splits, a.kvh, (groups + kHeads - 1) / kHeads),
+    auto kernel = chunk > kKeys ? awq_decode_attn_kernel<HD, true> : awq_decode_attn_kernel<HD, false>;
+    hipLaunchKernelGGL(kernel, dim3(splits, a.kvh, (groups + kHeads - 1) / kHeads),
                        dim3(kThreads), 0, stream, a.qkv, a.k_cache, a.v_cache, a.cos, a.sin, a.pos, a.part, a.nh,
                        a.kvh, groups, a.max_seq, chunk);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((awq_decode_combine_kernel<HD>), dim3(a.nh), dim3(4 * HD), 0, stream, a.part, a.pos, a.out,
-                       a.nh, a.max_seq, chunk);
+                       a.nh, a.max_seq, chunk, splits);
     return hipGetLastError();
 }
 
