@@ -31,7 +31,8 @@ namespace awq {
 //     loaded with the first k-step of each 128-row group only).
 // Each k-step runs in two phases that overlap the dequantisation of the next
 // k-half with the MFMAs of the current one (see the main loop).
-// FM: 16-row blocks per wave (8: 128 x rows per wave; 4: 64; 2: 32).
+// FM: 16-row blocks per wave (8: 128 x rows per wave; 4: 64; 2: 32; fewer where
+// M has fewer).
 // Variant 6 = FM 8: 128 x 256 tiles, two workgroups per CU, last-arriver
 // split-K finish; 7, 8, 9 = FM 8, 4, 2: 128, 64 and 32 x 256 tiles (two,
 // three, four workgroups per CU) with the reduce-launch finish -- the smaller
@@ -57,10 +58,13 @@ struct T5Layout {
     static constexpr int WAVES = NW;
     // The ring, or the staged fp16 tile (rows BN x 2 + 32 bytes apart) if larger.
     static constexpr int SMEM = S * STAGE > BM * (BN * 2 + 32) ? S * STAGE : BM * (BN * 2 + 32);
-    static constexpr int X_LOADS = X_BYTES / 1024 / WAVES;  // dwordx4 loads per wave per stage (FM / 2)
+    static constexpr int X_BLOCKS = BM / 8;  // 8-row blocks of x, one dwordx4 load each
+    // Loads of x per wave and stage; where the blocks do not divide evenly the
+    // last waves load the last block again (the same bytes to the same place).
+    static constexpr int X_LOADS = (X_BLOCKS + WAVES - 1) / WAVES;
     // Workgroups per CU: by registers (accumulators 4 * FM float4 per lane)
     // and by LDS (S stages).
-    static constexpr int PER_CU_REG = NW == 8 ? 1 : (FM >= 8 ? 2 : (FM >= 4 ? 3 : 4));
+    static constexpr int PER_CU_REG = NW == 8 ? 1 : (FM >= 5 ? 2 : (FM >= 3 ? 3 : 4));
     static constexpr int PER_CU_LDS = (160 * 1024) / (SMEM + 64);
     static constexpr int PER_CU = PER_CU_REG < PER_CU_LDS ? PER_CU_REG : PER_CU_LDS;
     static constexpr int W_LOADS = 2;  // dwordx4 packed-weight loads per wave per stage (its own 2 KB)
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
     constexpr int BM = L::BM;
     constexpr int S = L::S;
     static_assert((S - 2) * L::LOADS <= 63, "vmcnt holds 6 bits");
-    static_assert(FM % 2 == 0 && L::X_LOADS >= 1, "a wave loads whole 8-row blocks of x");
+    static_assert(FM >= 2, "two B fragments are read ahead");
     static_assert(L::PER_CU >= 1 && L::PER_CU * L::SMEM <= 160 * 1024, "LDS per CU");
     static_assert(NW == 4 || (NW == 8 && FIN == 1 && !HY), "eight waves: reduce-launch finish only");
     __shared__ __attribute__((aligned(16))) unsigned char smem[L::SMEM];
@@ -190,13 +194,16 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
     const u32x4 rs = raw_rsrc(a.scales, (uint32_t)((size_t)(a.K / kGroup) * a.N * 2));
     const uint32_t lds0 = lds_addr(smem);
 
-    // x: load i of wave w writes rows 8 (X_LOADS w + i) .. + 7; lane l brings
+    // x: load i of wave w writes block X_LOADS w + i, rows 8 (X_LOADS w + i) ..
+    // + 7 (the last block where the waves do not divide them); lane l brings
     // row 8 b + l / 8, k-chunk (l % 8) ^ (l / 8) to LDS chunk position l % 8.
     // A row at or beyond M has an offset at or beyond the buffer's M x K x 2
     // bytes, so the range check zeroes it; load i's offset is load 0's plus
-    // 8 i rows.
+    // 8 i rows (uneven blocks: block 0's plus 8 rows per block).
+    constexpr bool X_EVEN = L::X_BLOCKS % NW == 0;
     const uint32_t x_voff =
-        (uint32_t)(((size_t)(m0 + 8 * L::X_LOADS * wave + (lane >> 3)) * a.K + 8 * ((lane & 7) ^ (lane >> 3))) * 2);
+        (uint32_t)(((size_t)(m0 + 8 * (X_EVEN ? L::X_LOADS * wave : 0) + (lane >> 3)) * a.K +
+                    8 * ((lane & 7) ^ (lane >> 3))) * 2);
     // Packed weights: wave w loads only its own packed columns 8 w .. 8 w + 7,
     // row-major (32 B a row): dwordx4 load i covers rows 32 i .. + 31, lane
     // l bringing the 16-byte slot (l % 2) ^ sw(r) (packed columns 4 s .. + 3)
@@ -243,9 +250,11 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
                                    zb + 32u);
         }
 #pragma unroll
-        for (int i = 0; i < L::X_LOADS; ++i)
-            buffer_load_lds_x4(rx, x_voff + (uint32_t)(16 * i) * (uint32_t)a.K, __builtin_amdgcn_readfirstlane((uint32_t)k0 * 2u),
-                               base + 1024u * (uint32_t)(L::X_LOADS * wave + i));
+        for (int i = 0; i < L::X_LOADS; ++i) {
+            const int b = X_EVEN ? L::X_LOADS * wave + i : min(L::X_LOADS * wave + i, L::X_BLOCKS - 1);
+            buffer_load_lds_x4(rx, x_voff + (uint32_t)(16 * (X_EVEN ? i : b)) * (uint32_t)a.K,
+                               __builtin_amdgcn_readfirstlane((uint32_t)k0 * 2u), base + 1024u * (uint32_t)b);
+        }
 #pragma unroll
         for (int i = 0; i < L::W_LOADS; ++i)
             buffer_load_lds_x4(rw, w_voff, __builtin_amdgcn_readfirstlane((uint32_t)(k0 + 32 * i) * (uint32_t)pn * 4u),
@@ -347,7 +356,7 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
         };
         // Phase 1 starts its dequantisation at chunk C0, once the reads it
         // issued in chunk 0 have had time to land.
-        constexpr int C0 = FM >= 8 ? 2 : 1;
+        constexpr int C0 = FM >= 7 ? 2 : 1;
         // KT is even (whole groups), so steps come in (even, odd) pairs: the
         // even step's loads bring the group's zero words and scales, and the
         // odd step's phase 1 forms the next group's splats.
@@ -682,6 +691,12 @@ int64_t tile_tiles(int M, int N, int variant) {
     return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 
+// The reduce-finish tile with FM 16-row blocks of x.
+template <int FM>
+static void tile_launch(const GemmArgs& a, const TileConfig& cfg, dim3 grid, uint32_t* counters, hipStream_t stream) {
+    hipLaunchKernelGGL((awq_tile_kernel<FM, 1>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters);
+}
+
 hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* counters, hipStream_t stream) {
     if (tile_variant_served(cfg.variant)) {
         const int64_t blocks = tile_hybrid(cfg.variant) ? cfg.grid : tile_tiles(a.M, a.N, cfg.variant) * cfg.split_k;
@@ -690,9 +705,31 @@ hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* count
         bool reduce = false;
         switch (cfg.variant) {
             case 6: hipLaunchKernelGGL((awq_tile_kernel<8, 0>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
-            case 7: hipLaunchKernelGGL((awq_tile_kernel<8, 1>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); reduce = true; break;
-            case 8: hipLaunchKernelGGL((awq_tile_kernel<4, 1>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); reduce = true; break;
-            case 9: hipLaunchKernelGGL((awq_tile_kernel<2, 1>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); reduce = true; break;
+            case 7:
+            case 8:
+            case 9: {
+                // A single tile of rows computes only the 16-row blocks that M
+                // has (the plan, the outputs' order of summation and the
+                // partials stay the same).  Measured in graphs, us, whole
+                // tile / trimmed: M = 77 on 3584 x 37888 44.4 / 39.6 and
+                // 18944 x 3584 27.4 / 24.5 (128 -> 80 rows); M = 48 31.9 / 30.7
+                // and 21.5 / 20.6 (64 -> 48).  16 rows instead of 32 gave nothing
+                // (12 decoder layers at M = 16: 727 us against 721).  Rings of 4
+                // and 6 stages were no faster at any of them and up to 11 % slower.
+                const int rows = tile5_rows(cfg.variant);
+                reduce = true;
+                switch (a.M <= rows ? (a.M + 15) / 16 : rows / 16) {
+                    case 1:
+                    case 2: tile_launch<2>(a, cfg, grid, counters, stream); break;
+                    case 3: tile_launch<3>(a, cfg, grid, counters, stream); break;
+                    case 4: tile_launch<4>(a, cfg, grid, counters, stream); break;
+                    case 5: tile_launch<5>(a, cfg, grid, counters, stream); break;
+                    case 6: tile_launch<6>(a, cfg, grid, counters, stream); break;
+                    case 7: tile_launch<7>(a, cfg, grid, counters, stream); break;
+                    default: tile_launch<8>(a, cfg, grid, counters, stream); break;
+                }
+                break;
+            }
             case 15: hipLaunchKernelGGL((awq_tile_kernel<8, 1, false, 8>), grid, dim3(512), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); reduce = true; break;
             case 13: hipLaunchKernelGGL((awq_tile_kernel<8, 0, true>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
             case 14: hipLaunchKernelGGL((awq_tile_kernel<4, 0, true>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
