@@ -785,9 +785,6 @@ int run_plan(const void* x, const int32_t* qweight, const int32_t* qzeros, const
              const void* norm_w = nullptr, float norm_eps = 0.0f) {
     if (M == 0) return AWQ_OK;
     GemmArgs a;
-    a.input = input;
-    a.norm_w = static_cast<const half_t*>(norm_w);
-    a.norm_eps = norm_eps;
     a.bias = static_cast<const half_t*>(bias);
     a.residual = static_cast<const half_t*>(residual);
     a.x = static_cast<const half_t*>(x);
@@ -829,6 +826,9 @@ int run_plan(const void* x, const int32_t* qweight, const int32_t* qzeros, const
         cfg.chunks_per_split = (int)((groups + p.split_k - 1) / p.split_k);
         cfg.depth = p.depth;
         cfg.cw = p.tile_n / 128;
+        cfg.input = input;
+        cfg.norm_w = static_cast<const half_t*>(norm_w);
+        cfg.norm_eps = norm_eps;
         a.partials = p.split_k > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + kPartialsOffset)
                                    : nullptr;
         e = launch_gemv(a, cfg, static_cast<uint32_t*>(workspace), s);

@@ -13,6 +13,7 @@
 // cut in place, see awq_device.h), the lanes accumulate
 // sum_r x[r] * (b + q[r]) and sum_r x[r], and each group folds
 // s * (that - (b + z) * sum_r x[r]) in fp32 once.
+#include <cstddef>
 #include <type_traits>
 
 #include "awq_kernels.h"
@@ -245,16 +246,67 @@ __global__ __launch_bounds__(512) void awq_gemv_stream_kernel(GemmArgs a, int ch
 // 7 KB from L2, and scales its own K range), kInputSiluMul takes SiLU(gate) *
 // up of its K range.  A launch in a replayed graph costs 2.1 us however small;
 // measured in graphs over 28 layers' weights, us, fused / two launches: norm
-// + 3584 x 4608 6.3 / 7.7, norm + 3584 x 37888 17.4 / 18.8, SiLU * up + 18944 x
-// 3584 11.4 / 13.5; a decoder layer 53.7 / 57.7.
+// + 3584 x 4608 6.3 / 7.7, norm + 3584 x 37888 17.3 / 18.6, SiLU * up + 18944 x
+// 3584 11.3 / 13.1; a decoder layer 53.7 / 57.7 (50 with the short lead below).
+//
+// The way to the first load.  At 5 us a call, the time before a workgroup's
+// first weight load counts: every kernel argument line is a cold scalar load,
+// and an integer division by an argument some 40 instructions (150 in 64
+// bits).  So the arguments are two 64-byte lines, the first holding all that
+// the loads need, divisors come with their reciprocals from the host, and
+// the launch's own dimensions come as arguments (the hidden ones lie in a
+// third line).  Measured in graphs over 450 MB of weights, us before / now, M
+// = 1, 3, 8: 3584 x 512 4.42 / 3.97, 5.57 / 5.06, 7.39 / 6.60; 3584 x 3584 5.35
+// / 4.88, 6.95 / 6.53, 8.98 / 8.11; 3584 x 18944 10.6 / 10.3, 13.2 / 12.9, 15.9
+// / 15.3; 18944 x 3584 10.8 / 10.5, 12.4 / 12.2, 14.5 / 14.1.
 constexpr int kQuadItemsPerThread = 4;  // prologue loads per thread (consts and x each)
 
-template <int MR, int D, bool NT, int CW, bool RED = false, int IN = kInputX>
-__global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int split_k, unsigned long long* fix) {
+constexpr int quad_x_items(int mr) { return mr > 8 ? 16 : (mr > 4 ? 8 : kQuadItemsPerThread); }
+
+struct QuadArgs {
+    const uint32_t* qweight;
+    const uint32_t* qzeros;
+    const half_t* scales;
+    const half_t* x;
+    int M, N, K;
+    uint32_t strips_waves;           // strips x 16 + waves per workgroup
+    uint32_t strips_inv;             // inverse(): see div_by
+    uint32_t split_k, split_inv;
+    uint32_t total;                  // workgroups
+    half_t* out;
+    const half_t* bias;
+    const half_t* residual;
+    unsigned long long* fix;
+    float* partials;
+    const half_t* norm_w;            // kInputNorm
+    float norm_eps;
+};
+static_assert(offsetof(QuadArgs, out) == 64 && sizeof(QuadArgs) <= 128, "two lines");
+
+static uint32_t inverse(uint32_t d) { return (uint32_t)((((uint64_t)1 << 31) + d - 1) / d); }
+// n / d and the remainder for n < 2^31, inv = inverse(d) = ceil(2^31 / d): inv
+// exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less
+// than n / 2^31 and is at most one too large.
+__device__ __forceinline__ uint32_t div_by(uint32_t n, uint32_t d, uint32_t inv, uint32_t& rem) {
+    uint32_t q = __umulhi(2u * n, inv);
+    q -= q * d > n ? 1u : 0u;
+    rem = n - q * d;
+    return q;
+}
+
+// ONE: a workgroup has no more zero words and pieces of x to stage than
+// threads (most split plans): one prologue load of each per thread.
+template <int MR, int D, bool NT, int CW, bool RED = false, int IN = kInputX, bool ONE = false>
+__global__ __launch_bounds__(512) void awq_gemv_quad_kernel(QuadArgs a) {
     extern __shared__ __align__(16) uint32_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nw = blockDim.x >> 6;
+    // One wait for the whole first line of arguments.
+    asm volatile("" ::"s"(a.qweight), "s"(a.qzeros), "s"(a.scales), "s"(a.x), "s"(a.M), "s"(a.N), "s"(a.K),
+                 "s"(a.strips_waves), "s"(a.strips_inv), "s"(a.split_k), "s"(a.split_inv), "s"(a.total));
+    const int nw = (int)(a.strips_waves & 15u);
+    const uint32_t n_strips = a.strips_waves >> 4;
+    const int split_k = (int)a.split_k;
     const int c4 = lane & 15;
     const int rq = lane >> 4;
     constexpr int SP = 16 * CW;  // packed columns of a strip
@@ -262,30 +314,30 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
     // D rows live per lane: MR <= 4, rows 0 .. MR - 1 in the lanes of k-block
     // 0; MR = 8 / 16, rows 4 rq .. 4 rq + 3 in the lanes of k-blocks 0 .. 1 / 0 .. 3.
     constexpr int NR = MR > 4 ? 4 : MR;
-    constexpr int XI = MR > 8 ? 16 : (MR > 4 ? 8 : kQuadItemsPerThread);  // x prologue loads per thread
+    constexpr int XI = ONE ? 1 : quad_x_items(MR);                    // x prologue loads per thread
+    constexpr int CI = ONE ? 1 : kQuadItemsPerThread;                 // zero words and scales
     static_assert(MR <= 8 || RED, "16 rows of x take the reduce-launch finish");
     static_assert(IN == kInputX || MR == 1, "a made input is one row");
     const int pn = a.N >> 3;
-    const int n_strips = (pn + SP - 1) / SP;
     // Work item w = (split, strip), strip fastest, numbered in XCD order:
     // workgroups are dispatched round-robin over the 8 XCDs (workgroup b on
     // XCD b % 8), and the workgroups one XCD runs get consecutive items, so
     // neighbouring strips run on one XCD -- with 128-column strips (64-byte
     // row segments) two strips share each 128-byte line, which one L2 then
     // fetches once.  Any numbering is correct; this one is about traffic.
-    const int total = (int)gridDim.x;
-    const int xb = (int)blockIdx.x & 7, xi = (int)blockIdx.x >> 3, per_x = (total + 7) >> 3, rem_x = total & 7;
-    const int w_item = (rem_x == 0 || xb < rem_x) ? xb * per_x + xi : rem_x * per_x + (xb - rem_x) * (per_x - 1) + xi;
-    const int strip = w_item % n_strips;
-    const int split = w_item / n_strips;
+    const int xb = (int)blockIdx.x & 7, xi = (int)blockIdx.x >> 3;
+    const int w_item = xb * (int)(a.total >> 3) + min(xb, (int)(a.total & 7u)) + xi;
+    uint32_t strip_u, rem;
+    const uint32_t split = div_by((uint32_t)w_item, n_strips, a.strips_inv, strip_u);
+    const int strip = (int)strip_u;
     const int jl = min(strip * SP + CW * c4, pn - CW);  // in-range columns; lanes past pn drop their results
-    const int C = a.K / 32;
-    const int c0 = (int)((int64_t)C * split / split_k);
-    const int c1 = (int)((int64_t)C * (split + 1) / split_k);
+    const uint32_t C = (uint32_t)a.K / 32u;  // C x split_k < 2^26
+    const int c0 = (int)div_by(C * split, a.split_k, a.split_inv, rem);
+    const int c1 = (int)div_by(C * (split + 1u), a.split_k, a.split_inv, rem);
     const int nc = c1 - c0;
     const int g_lo = c0 / 4;
     const int n_g = nc > 0 ? (c1 - 1) / 4 - g_lo + 1 : 0;
-    const int groups = a.K / kGroup;
+    const int groups = (int)((uint32_t)a.K / (uint32_t)kGroup);
 
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.qweight, (uint32_t)((size_t)a.K * pn * 4));
     const __amdgpu_buffer_rsrc_t rz = make_rsrc(a.qzeros, (uint32_t)((size_t)groups * pn * 4));
@@ -303,25 +355,42 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
 
     // Prologue loads: item (g, j) = zero word and 8 scales of packed column j
     // of group g_lo + g; x in 16-byte pieces.  Issued before the weights.
-    const int nt = blockDim.x;
-    u32x4 sv[kQuadItemsPerThread];
-    uint32_t zv[kQuadItemsPerThread];
+    const int nt = 64 * nw;
+    u32x4 sv[CI];
+    uint32_t zv[CI];
     u32x4 xv[XI];
     auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
 #pragma unroll
-    for (int i = 0; i < kQuadItemsPerThread; ++i) {
-        const int item = min((int)threadIdx.x + i * nt, max(n_g * SP - 1, 0));
+    for (int i = 0; i < CI; ++i) {
+        // Items past the last read out of range, without memory traffic; a
+        // branch around them would make the wave wait for the loads before it.
+        const int item = (int)threadIdx.x + i * nt;
         const int g = g_lo + item / SP;
         const int j = min(strip * SP + item % SP, pn - 1);
-        zv[i] = buf_load_b32(rz, (uint32_t)(g * pn + j) * 4u, 0u);
-        sv[i] = buf_load_u4(rs, (uint32_t)(((size_t)g * a.N + 8 * j) * 2), 0u);
+        const uint32_t word = (uint32_t)(g * pn + j);
+        zv[i] = buf_load_b32(rz, item < n_g * SP ? word * 4u : 0x80000000u, 0u);
+        sv[i] = buf_load_u4(rs, item < n_g * SP ? word * 16u : 0x80000000u, 0u);
     }
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
         const int xi = (int)threadIdx.x + i * nt;  // x piece: row m, 8 rows at c0*32 + 8 * (xi % (nc * 4))
-        const int m = xi / max(nc * 4, 1);
-        const uint32_t xoff = (uint32_t)(((size_t)m * a.K + (size_t)c0 * 32 + 8 * (xi % max(nc * 4, 1))) * 2);
-        xv[i] = buf_load_u4(rx, m < MR ? xoff : 0x80000000u, 0u);
+        int m = 0, piece = xi;
+        if constexpr (MR > 1) {
+            // m = xi / (nc * 4) by a float reciprocal, exact after one step
+            // either way (xi < 2^13).
+            const int per = max(nc * 4, 1);
+            m = (int)((float)xi * __builtin_amdgcn_rcpf((float)per));
+            piece = xi - m * per;
+            if (piece < 0) {
+                --m;
+                piece += per;
+            } else if (piece >= per) {
+                ++m;
+                piece -= per;
+            }
+        }
+        const uint32_t xoff = (uint32_t)(((size_t)m * a.K + (size_t)c0 * 32 + 8 * piece) * 2);
+        xv[i] = buf_load_u4(rx, (MR > 1 ? m < MR : xi < nc * 4) ? xoff : 0x80000000u, 0u);
     }
     // The made inputs' other operand (the norm's weight or up), and for the
     // norm the whole row (pieces past it read zeros).
@@ -382,7 +451,7 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
     fence();
 
 #pragma unroll
-    for (int i = 0; i < kQuadItemsPerThread; ++i) {
+    for (int i = 0; i < CI; ++i) {
         const int item = (int)threadIdx.x + i * nt;
         if (item < n_g * SP) {
             const int g = item / SP;
@@ -558,7 +627,7 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(GemmArgs a, int spli
                 fn[i * FB + mm] = strip * SC + t;
                 fok[i * FB + mm] = t < SC && strip * SC + t < a.N && m < a.M;
             }
-        finish_batch<kOwn * FB>(fix, a.out, a.bias, a.residual, a.M, a.N, split_k, fs, fm, fn, fok);
+        finish_batch<kOwn * FB>(a.fix, a.out, a.bias, a.residual, a.M, a.N, split_k, fs, fm, fn, fok);
     }
 }
 
@@ -591,7 +660,7 @@ bool gemv_quad_fits(int M, int K, int split_k, int k_waves, int cw) {
     const int64_t threads = 64 * (int64_t)k_waves;
     const int mr = gemv_quad_mr(M);
     return gemv_quad_max_groups(K, split_k) * 16 * cw <= kQuadItemsPerThread * threads &&
-           mr * per * 4 <= (mr > 8 ? 16 : (mr > 4 ? 8 : kQuadItemsPerThread)) * threads;
+           mr * per * 4 <= quad_x_items(mr) * threads;
 }
 
 int64_t gemv_strips(int N) { return ((N >> 3) + 63) / 64; }
@@ -611,17 +680,45 @@ int gemv_norm_max_k(int k_waves) { return kQuadItemsPerThread * 64 * k_waves * 8
 template <int MR, int D, int CW, bool RED = false, int IN = kInputX>
 static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uint32_t* counters,
                                    hipStream_t stream) {
-    unsigned long long* fix = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(counters) + kCounterBytes);
     const size_t lds = gemv_quad_lds_bytes(a.M, a.K, cfg.split_k, cfg.kw_count, CW);
-    const dim3 grid((unsigned)(gemv_strips_cw(a.N, CW) * cfg.split_k)), block(64 * cfg.kw_count);
+    const uint32_t strips = (uint32_t)gemv_strips_cw(a.N, CW);
+    const dim3 grid(strips * (uint32_t)cfg.split_k), block(64 * cfg.kw_count);
+    QuadArgs q;
+    q.qweight = a.qweight;
+    q.qzeros = a.qzeros;
+    q.scales = a.scales;
+    q.x = a.x;
+    q.M = a.M;
+    q.N = a.N;
+    q.K = a.K;
+    q.strips_waves = strips * 16u + (uint32_t)cfg.kw_count;  // at most 8 waves
+    q.strips_inv = inverse(strips);
+    q.split_k = (uint32_t)cfg.split_k;
+    q.split_inv = inverse(q.split_k);
+    q.out = a.out;
+    q.bias = a.bias;
+    q.residual = a.residual;
+    q.fix = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(counters) + kCounterBytes);
+    q.partials = a.partials;
+    q.norm_w = cfg.norm_w;
+    q.norm_eps = cfg.norm_eps;
+    q.total = grid.x;
     // Weight loads marked non-temporal where each workgroup streams a long
     // K range (few splits): 3584 x 37888 at split 3 measured 2.7 - 4.7 %
     // faster with them at M = 1 - 16, the 100 - 500-row ranges of 18 - 36
     // splits up to 3 % slower.
-    if (cfg.split_k <= kNonTemporalMaxSplit)
-        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, true, CW, RED, IN>), grid, block, lds, stream, a, cfg.split_k, fix);
-    else
-        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, false, CW, RED, IN>), grid, block, lds, stream, a, cfg.split_k, fix);
+    if (cfg.split_k <= kNonTemporalMaxSplit) {
+        hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, true, CW, RED, IN>), grid, block, lds, stream, q);
+    } else {
+        const int64_t per = (a.K / 32 + cfg.split_k - 1) / cfg.split_k;
+        const bool one = gemv_quad_max_groups(a.K, cfg.split_k) * 16 * CW <= (int64_t)block.x &&
+                         MR * per * 4 <= (int64_t)block.x;
+        if (D == 2 && CW == 1 && MR <= 8 && one)
+            hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, false, CW, RED, IN, D == 2 && CW == 1 && MR <= 8>), grid,
+                               block, lds, stream, q);
+        else
+            hipLaunchKernelGGL((awq_gemv_quad_kernel<MR, D, false, CW, RED, IN>), grid, block, lds, stream, q);
+    }
     const hipError_t e = hipGetLastError();
     if (!RED || e != hipSuccess || cfg.split_k <= 1) return e;
     return splitk_reduce_launch(a, cfg.split_k, stream);
@@ -641,8 +738,8 @@ static hipError_t gemv_quad_input_dispatch(const GemmArgs& a, const GemvConfig& 
 
 static hipError_t gemv_quad_dispatch(const GemmArgs& a, const GemvConfig& cfg, uint32_t* counters,
                                      hipStream_t stream) {
-    if (a.input == kInputNorm) return gemv_quad_input_dispatch<kInputNorm>(a, cfg, counters, stream);
-    if (a.input == kInputSiluMul) return gemv_quad_input_dispatch<kInputSiluMul>(a, cfg, counters, stream);
+    if (cfg.input == kInputNorm) return gemv_quad_input_dispatch<kInputNorm>(a, cfg, counters, stream);
+    if (cfg.input == kInputSiluMul) return gemv_quad_input_dispatch<kInputSiluMul>(a, cfg, counters, stream);
     if (cfg.cw == 1) {
         switch (gemv_quad_mr(a.M) * 10 + cfg.depth) {
             case 12: return gemv_quad_launch<1, 2, 1>(a, cfg, counters, stream);

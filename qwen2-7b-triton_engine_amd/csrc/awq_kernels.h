@@ -20,11 +20,6 @@ struct GemmArgs {
     int M, N, K;
     const half_t* bias = nullptr;      // [N] added to every row (epilogue), or null
     const half_t* residual = nullptr;  // [M, N] added after the bias (epilogue), or null; may alias out
-    // How the decode GEMV's prologue makes its row of x (kInput*; M == 1,
-    // launch_gemv variant 5 with depth 2 only; every other launch takes kInputX).
-    int input = 0;
-    const half_t* norm_w = nullptr;    // kInputNorm: [K]
-    float norm_eps = 0.0f;
 };
 // x is the row; x is normalised on the way: fp16(x * rsqrt(mean(x^2) + eps) *
 // w); x is gate||up [2 K] and the row is fp16(silu(gate) * up).
@@ -48,6 +43,11 @@ struct GemvConfig {
     int chunks_per_split;    // variant 2: 128-row groups per workgroup
     int depth;               // variant 2: chunk buffers in flight (2, 3 or 4; 4 only for 16 rows per wave)
     int cw;                  // variant 5: packed columns per lane, 4 (512-column strips) or 2 (256)
+    // How the prologue makes its row of x (kInput*; M == 1, variant 5 with
+    // depth 2 only).
+    int input = kInputX;
+    const half_t* norm_w = nullptr;  // kInputNorm: [K]
+    float norm_eps = 0.0f;
 };
 
 // Tile variants 6 .. 9, 13, 14, 15: weights dequantised into MFMA registers,
