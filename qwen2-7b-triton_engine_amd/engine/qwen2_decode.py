@@ -12,7 +12,10 @@ in torch, in fp32 on contiguous operands), RMSNorm (``:15-22``) in
 ``kernels.rmsnorm``, and the embedding lookup in torch.  The QKV bias and
 the residual adds after o_proj and down_proj run in the GEMM's epilogue,
 and SiLU * up reads the fused gate||up output in one kernel
-(``kernels.silu_mul``).  Logits are computed for the last position only, where the
+(``kernels.silu_mul``); a decode step's norms and SiLU * up run in the next
+projection's prologue.  A layer is one call into the torch binding
+(``qwen2_layer``), which issues all of this; models that the kernels do not
+serve take the same steps from here.  Logits are computed for the last position only, where the
 reference computes them for every position and keeps the last
 (``inference/engine.py:93,127``).
 
@@ -30,9 +33,9 @@ import time
 
 import torch
 
+from kernels import _native
 from kernels.attention import attention_decode, attention_prefill, attention_served
-from kernels._native import INPUT_RMSNORM, INPUT_SILU_MUL
-from kernels.awq_gemm import awq_gemm_decode, awq_gemm_forward, awq_gemm_forward_ex, decode_linear_served
+from kernels.awq_gemm import awq_gemm_forward, awq_gemm_forward_ex
 from kernels.lm_head import lm_head_forward
 from kernels.rmsnorm import MAX_H, rmsnorm
 from kernels.silu_mul import silu_mul_gate_up
@@ -162,6 +165,10 @@ class Qwen2AwqDecoder:
         self.v_cache = torch.zeros_like(self.k_cache)
         # the HIP attention serves heads of 64 or 128 columns; torch the others
         self._hip_attention = attention_served(shape.num_heads, KV, hd, max_seq_len)
+        # the whole layer in one native call: heads and rows that the kernels
+        # serve, and this class's own projections
+        self._native_layers = (self._hip_attention and H <= MAX_H and H % 8 == 0 and
+                               type(self).linear is Qwen2AwqDecoder.linear)
         self._graph = None
 
     # ---- linear layers: the path this build replaces -------------------------
@@ -176,23 +183,17 @@ class Qwen2AwqDecoder:
     # ---- one decoder layer over positions `pos` (device int64 [S]) -------------
     def _layer(self, li: int, h: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         p = self.layers[li]
-        qkv = self._normed_linear(h, p["ln1"], p["qkv"], bias=p["qkv_bias"])
+        if self._native_layers and all(
+                getattr(p[k], "dtype", None) is torch.float16 for k in ("ln1", "ln2", "qkv_bias")):
+            return _native.binding().qwen2_layer(h, pos, causal, p, self.k_cache[li], self.v_cache[li], self.cos,
+                                                 self.sin, self.s.num_heads, self.s.rms_norm_eps)
+        x = _rmsnorm(h, p["ln1"], self.s.rms_norm_eps)
+        qkv = self.linear(x, p["qkv"], bias=p["qkv_bias"])
         att = self._attention(li, qkv, pos, causal)
         h = self.linear(att, p["o"], residual=h)
-        gate_up = self._normed_linear(h, p["ln2"], p["gate_up"])
-        if self._one_row(gate_up, p["down"], INPUT_SILU_MUL):
-            return awq_gemm_decode(INPUT_SILU_MUL, gate_up, *p["down"], residual=h)
-        return self.linear(silu_mul_gate_up(gate_up), p["down"], residual=h)
-
-    def _one_row(self, x: torch.Tensor, op, kind: int) -> bool:
-        """Whether this is a decode row that the projection `op` makes its input of."""
-        return x.shape[0] == 1 and decode_linear_served(op[2].shape[1], op[0].shape[0], kind)
-
-    def _normed_linear(self, h: torch.Tensor, w: torch.Tensor, op, bias: torch.Tensor | None = None) -> torch.Tensor:
-        """The projection `op` of RMSNorm(h)."""
-        if w.dtype == torch.float16 and h.dtype == torch.float16 and self._one_row(h, op, INPUT_RMSNORM):
-            return awq_gemm_decode(INPUT_RMSNORM, h, *op, norm_w=w, eps=self.s.rms_norm_eps, bias=bias)
-        return self.linear(_rmsnorm(h, w, self.s.rms_norm_eps), op, bias=bias)
+        x = _rmsnorm(h, p["ln2"], self.s.rms_norm_eps)
+        inter = silu_mul_gate_up(self.linear(x, p["gate_up"]))
+        return self.linear(inter, p["down"], residual=h)
 
     def _attention(self, li: int, qkv: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         """Attention output fp16 [S, heads * head_dim] of the positions `pos`,
@@ -255,7 +256,9 @@ class Qwen2AwqDecoder:
         """One eager decode step: logits after feeding `token` at position `pos`."""
         if not 0 <= pos < self.max_seq_len:
             raise ValueError(f"position {pos} outside [0, {self.max_seq_len})")
-        return self._forward(token.view(1).to(self.dev), torch.tensor([pos], device=self.dev), causal=False)
+        # filled on the device: a tensor made from host data would wait for the stream
+        where = torch.full((1,), pos, dtype=torch.int64, device=self.dev)
+        return self._forward(token.view(1).to(self.dev), where, causal=False)
 
     @torch.no_grad()
     def _capture(self):

@@ -243,6 +243,11 @@ def awq_gemm_forward_ex(x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Te
     ``bias`` fp16 ``[N]`` (``out + bias``, model/qwen2.py:45-46,108-109) and
     ``residual`` fp16 ``[..., N]`` (``residual + out``, :219-227), bit-identical
     to the unfused torch adds.  ``residual`` may be ``out`` itself."""
+    if path is None and plan_obj is None and out is None:
+        try:    # the AUTO plan into a new tensor: one call into the torch binding
+            return _native.binding().gemm(x, qweight, qzeros, scales, group_size, bias, residual)
+        except RuntimeError:
+            pass    # a refused plan or launch: the calls below raise it with its status
     in_shape, x_flat, qweight, qzeros, scales, K, N, dev = _prepare(x, qweight, qzeros, scales, group_size)
     M = x_flat.shape[0]
     if out is None:
