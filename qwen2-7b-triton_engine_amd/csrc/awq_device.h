@@ -211,6 +211,18 @@ __device__ __forceinline__ void wait_batches(int n) {
     }
 }
 
+// Division by a kernel argument whose reciprocal the host passes: n / d and
+// the remainder for n < 2^31, inv = div_inverse(d) = ceil(2^31 / d).  inv
+// exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less
+// than n / 2^31 and is at most one too large.
+inline uint32_t div_inverse(uint32_t d) { return (uint32_t)((((uint64_t)1 << 31) + d - 1) / d); }
+__device__ __forceinline__ uint32_t div_by(uint32_t n, uint32_t d, uint32_t inv, uint32_t& rem) {
+    uint32_t q = __umulhi(2u * n, inv);
+    q -= q * d > n ? 1u : 0u;
+    rem = n - q * d;
+    return q;
+}
+
 // Device-scope (cache policy SC1) 16-byte store and load: coherent across
 // the XCDs of the device without whole-L2 maintenance.
 constexpr int kCpolSC1 = 16;
@@ -295,6 +307,21 @@ __device__ __forceinline__ void store_out(half_t* out, const half_t* bias, const
         static_assert(V == 4, "4 or 8 outputs");
         typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, h), ro, (uint32_t)(o * 2), 0, kCpolSC1);
+    }
+}
+// V consecutive values of an epilogue operand (bias or residual; zeros if it
+// is null) in one load, where its address allows that -- C callers may pass
+// any 2-byte aligned one.
+template <int V>
+__device__ __forceinline__ void load_epi(const half_t* p, half_t (&v)[V]) {
+    typedef _Float16 hv_t __attribute__((ext_vector_type(V)));
+    if (p != nullptr && (reinterpret_cast<uintptr_t>(p) & (2 * V - 1)) == 0) {
+        const hv_t h = *reinterpret_cast<const hv_t*>(p);
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = h[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = p != nullptr ? p[i] : (half_t)0;
     }
 }
 // epi_round with the bias / residual values already loaded (has_* says

@@ -270,7 +270,7 @@ struct QuadArgs {
     const half_t* x;
     int M, N, K;
     uint32_t strips_waves;           // strips x 16 + waves per workgroup
-    uint32_t strips_inv;             // inverse(): see div_by
+    uint32_t strips_inv;             // div_inverse
     uint32_t split_k, split_inv;
     uint32_t total;                  // workgroups
     half_t* out;
@@ -282,17 +282,6 @@ struct QuadArgs {
     float norm_eps;
 };
 static_assert(offsetof(QuadArgs, out) == 64 && sizeof(QuadArgs) <= 128, "two lines");
-
-static uint32_t inverse(uint32_t d) { return (uint32_t)((((uint64_t)1 << 31) + d - 1) / d); }
-// n / d and the remainder for n < 2^31, inv = inverse(d) = ceil(2^31 / d): inv
-// exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less
-// than n / 2^31 and is at most one too large.
-__device__ __forceinline__ uint32_t div_by(uint32_t n, uint32_t d, uint32_t inv, uint32_t& rem) {
-    uint32_t q = __umulhi(2u * n, inv);
-    q -= q * d > n ? 1u : 0u;
-    rem = n - q * d;
-    return q;
-}
 
 // ONE: a workgroup has no more zero words and pieces of x to stage than
 // threads (most split plans): one prologue load of each per thread.
@@ -692,9 +681,9 @@ static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uin
     q.N = a.N;
     q.K = a.K;
     q.strips_waves = strips * 16u + (uint32_t)cfg.kw_count;  // at most 8 waves
-    q.strips_inv = inverse(strips);
+    q.strips_inv = div_inverse(strips);
     q.split_k = (uint32_t)cfg.split_k;
-    q.split_inv = inverse(q.split_k);
+    q.split_inv = div_inverse(q.split_k);
     q.out = a.out;
     q.bias = a.bias;
     q.residual = a.residual;

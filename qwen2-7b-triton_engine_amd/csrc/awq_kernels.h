@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/awq_w4a16.h"
 #include "awq_device.h"
 
@@ -171,9 +173,47 @@ int64_t stream_threads(int layout, int k_waves);
 hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* counters, hipStream_t stream);
 int64_t tile_tiles(int M, int N, int variant);
 uint64_t tile_partials_bytes(int64_t split_k, int64_t M, int64_t N);
-// Threads that share one output piece in the reduce launches (enough that
-// each adds at most eight splits; eight from 12 splits up).
-int stream_reduce_parts(int split_k);
+// Threads that share one output piece in the reduce launches: enough that
+// each adds at most eight splits, and eight from 12 splits up -- measured
+// behind the 32-row tile at M = 8 and 16 (14 and 28 splits) 0.5 - 1.25 us
+// faster than two or four, with no change at 36 splits (already eight) or at
+// 3 (one).
+inline int stream_reduce_parts(int split_k) {
+    int P = 1;
+    while (P < 16 && P * 8 < split_k) P *= 2;
+    if (split_k >= 12 && P < 8) P = 8;
+    return P;
+}
+// f(threads per piece, splits loaded at a time) with both as constants: the
+// smallest instance that covers ceil(split_k / threads) splits in one go
+// (more splits loop).  Loads past the last split cost their instructions, so
+// eight for every count was slower than the loop it replaced where the
+// partials are large (o_proj at M = 300: 23.9 us against 23.4).
+template <typename F>
+void with_reduce_shape(int split_k, F f) {
+    const int parts = stream_reduce_parts(split_k), each = (split_k + parts - 1) / parts;
+    using std::integral_constant;
+    constexpr integral_constant<int, 1> c1;
+    constexpr integral_constant<int, 2> c2;
+    constexpr integral_constant<int, 3> c3;
+    constexpr integral_constant<int, 4> c4;
+    constexpr integral_constant<int, 8> c8;
+    constexpr integral_constant<int, 16> c16;
+    if (parts == 1) {
+        if (each <= 2) f(c1, c2);
+        else if (each == 3) f(c1, c3);
+        else if (each == 4) f(c1, c4);
+        else f(c1, c8);
+    } else if (parts == 2) {
+        f(c2, c8);
+    } else if (parts <= 8) {     // four threads are never chosen: 17 splits and more take eight
+        if (each <= 2) f(c8, c2);
+        else if (each <= 4) f(c8, c4);
+        else f(c8, c8);
+    } else {
+        f(c16, c8);
+    }
+}
 
 // Output columns per skinny wave.
 constexpr int kSkinnyCols = 128;

@@ -461,31 +461,62 @@ __global__ __launch_bounds__(R == 2 ? 512 : 256) void awq_stream_kernel(GemmArgs
 // all in flight together) and combine through LDS in part order.  The
 // partials are read once and left as they are (the workspace's partials
 // region is not kept zero).
-__global__ __launch_bounds__(256) void awq_splitk_reduce_kernel(float* __restrict__ partials, half_t* __restrict__ out,
-                                                               const half_t* bias, const half_t* residual, int M,
-                                                               int N, int split_k, int P) {
+//
+// Bound by latency (a few MB, 3 - 4 us): all arguments are one line read with
+// one wait, P is a constant, a thread's splits load U at a time (past the
+// last: out of range, no traffic) together with the epilogue's operands.
+struct ReduceArgs {
+    const float* partials;
+    half_t* out;
+    const half_t* bias;
+    const half_t* residual;
+    uint32_t M, N, split_k, quads_per_row, inv;  // N / 4 and its div_inverse
+};
+static_assert(sizeof(ReduceArgs) <= 64, "one line");
+template <int P, int U>
+__global__ __launch_bounds__(256) void awq_splitk_reduce_kernel(ReduceArgs a) {
+    asm volatile("" ::"s"(a.partials), "s"(a.out), "s"(a.bias), "s"(a.residual), "s"(a.M), "s"(a.N), "s"(a.split_k),
+                 "s"(a.quads_per_row), "s"(a.inv));
     __shared__ floatx4 fin[256];
-    const int qpb = 256 / P;  // output quads per workgroup
+    constexpr int kQuads = 256 / P;  // output quads per workgroup
     const int t = threadIdx.x;
-    const int part = t / qpb;
-    const int quads = M * N / 4;
-    const int q = blockIdx.x * qpb + t % qpb;
+    const int part = t / kQuads;
+    const uint32_t q = blockIdx.x * kQuads + t % kQuads, quads = a.M * a.quads_per_row;
     const bool valid = q < quads;
-    const size_t stride = (size_t)M * N;
-    floatx4 s = {0.f, 0.f, 0.f, 0.f};
-    if (valid) {
-        floatx4* p = reinterpret_cast<floatx4*>(partials) + q;
-        const size_t step = stride / 4;  // one split, in float4
-#pragma unroll 8
-        for (int sp = part; sp < split_k; sp += P) s += __builtin_nontemporal_load(p + (size_t)sp * step);
+    const uint32_t step = quads * 16u;  // bytes of one split; split_k of them are below 2^31
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.partials, a.split_k * step);
+    uint32_t col;
+    const uint32_t m = div_by(valid ? q : 0u, a.quads_per_row, a.inv, col);
+    half_t bv[4], rv[4];
+    if (part == 0) {
+        load_epi<4>(a.bias ? a.bias + 4 * col : nullptr, bv);
+        load_epi<4>(a.residual ? a.residual + (size_t)m * a.N + 4 * col : nullptr, rv);
     }
-    fin[t] = s;
-    __syncthreads();
+    floatx4 s = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t s0 = part; s0 < a.split_k; s0 += U * P) {
+        u32x4 v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const uint32_t sp = s0 + i * P;
+            v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 rp, valid && sp < a.split_k ? sp * step + q * 16u : 0x80000000u, 0u, kCpolNT));
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) s += __builtin_bit_cast(floatx4, v[i]);
+    }
+    if constexpr (P > 1) {
+        fin[t] = s;
+        __syncthreads();
+    }
     if (valid && part == 0) {
-        for (int i = 1; i < P; ++i) s += fin[i * qpb + t];
-        const float y[4] = {s[0], s[1], s[2], s[3]};
-        const int m = (int)(((size_t)q * 4) / N);
-        store_out<4>(out, bias, residual, N, m, q * 4 - m * N, y);
+#pragma unroll
+        for (int i = 1; i < P; ++i) s += fin[i * kQuads + t];
+        typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+        h4_t h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = epi_round_vals(s[i], a.bias != nullptr, bv[i], a.residual != nullptr, rv[i]);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, h), make_rsrc(a.out, 0x7FFFFFFFu), q * 8u, 0,
+                                              kCpolSC1);
     }
 }
 
@@ -507,26 +538,20 @@ bool stream_fits(int M, int K, int split_k, int k_waves, int layout) {
     return split_k <= groups && n_g * 64 <= items && (layout != kStreamRowLayout || (int64_t)M * n_g * 16 <= items);
 }
 
-// Threads per output quad of the reduce launch: enough that each adds at
-// most eight splits, and eight from 12 splits up -- measured behind the
-// 32-row tile at M = 8 and 16 (14 and 28 splits) 0.5 - 1.25 us faster than
-// two or four, with no change at 36 splits (already eight) or at 3 (one).
-int stream_reduce_parts(int split_k) {
-    int P = 1;
-    while (P < 16 && P * 8 < split_k) P *= 2;
-    if (split_k >= 12 && P < 8) P = 8;
-    return P;
-}
-
 int64_t stream_reduce_blocks(int M, int N, int split_k) {
     const int64_t qpb = 256 / stream_reduce_parts(split_k);
     return ((int64_t)M * N / 4 + qpb - 1) / qpb;
 }
 
 hipError_t splitk_reduce_launch(const GemmArgs& a, int split_k, hipStream_t stream) {
-    const int P = stream_reduce_parts(split_k);
-    hipLaunchKernelGGL(awq_splitk_reduce_kernel, dim3((unsigned)stream_reduce_blocks(a.M, a.N, split_k)), dim3(256), 0,
-                       stream, a.partials, a.out, a.bias, a.residual, a.M, a.N, split_k, P);
+    const uint32_t row = (uint32_t)a.N / 4;
+    const ReduceArgs r{a.partials, a.out, a.bias, a.residual, (uint32_t)a.M, (uint32_t)a.N, (uint32_t)split_k, row,
+                       div_inverse(row)};
+    const dim3 grid((unsigned)stream_reduce_blocks(a.M, a.N, split_k)), block(256);
+    with_reduce_shape(split_k, [&](auto parts, auto unroll) {
+        hipLaunchKernelGGL((awq_splitk_reduce_kernel<decltype(parts)::value, decltype(unroll)::value>), grid, block, 0,
+                           stream, r);
+    });
     return hipGetLastError();
 }
 

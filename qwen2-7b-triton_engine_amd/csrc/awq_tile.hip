@@ -637,42 +637,76 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
 // (even and odd columns).  P threads share such a piece (splits p, p + P,
 // ...; at most eight splits each) and combine
 // through LDS in part order.  32 consecutive threads read one kilobyte.
-__global__ __launch_bounds__(256) void awq_tile_reduce_kernel(const float* __restrict__ partials, half_t* __restrict__ out,
-                                                             const half_t* bias, const half_t* residual, int M, int N,
-                                                             int split_k, int P) {
+// Latency, as awq_splitk_reduce_kernel: one line of arguments, P a constant,
+// U splits' loads in flight (past the last: out of range), the epilogue's
+// operands loaded with them.
+struct TileReduceArgs {
+    const float* partials;
+    half_t* out;
+    const half_t* bias;
+    const half_t* residual;
+    uint32_t M, N, split_k, nt, nt_inv, units;  // column tiles and their div_inverse; units: 16-row blocks x nt
+};
+static_assert(sizeof(TileReduceArgs) <= 64, "one line");
+template <int P, int U>
+__global__ __launch_bounds__(256) void awq_tile_reduce_kernel(TileReduceArgs a) {
+    asm volatile("" ::"s"(a.partials), "s"(a.out), "s"(a.bias), "s"(a.residual), "s"(a.M), "s"(a.N), "s"(a.split_k),
+                 "s"(a.nt), "s"(a.nt_inv), "s"(a.units));
     __shared__ floatx4 fin[2][256];
-    const int per_wg = 256 / P;  // pieces per workgroup
+    constexpr int kPieces = 256 / P;  // pieces per workgroup
     const int t = threadIdx.x;
-    const int part = t / per_wg;
-    const int RB = (M + 15) >> 4, NT = (N + T5_BN - 1) / T5_BN;
-    const int piece = blockIdx.x * per_wg + t % per_wg;
-    const int u = piece >> 9, in = piece & 511;     // unit rb x NT + tn; 512 pieces a unit
-    const int wc = in >> 5, j = (in >> 4) & 1, n16 = in & 15;
-    const int rb = u / NT, tn = u - rb * NT;
-    const int m = 16 * rb + n16;
-    const int n = T5_BN * tn + 64 * (wc >> 2) + 16 * (wc & 3) + 8 * j;
-    const bool valid = u < RB * NT && m < M && n < N;
+    const int part = t / kPieces;
+    const uint32_t piece = blockIdx.x * kPieces + t % kPieces;
+    const uint32_t u = piece >> 9, in = piece & 511u;  // unit rb x nt + tn; 512 pieces a unit
+    const uint32_t wc = in >> 5, j = (in >> 4) & 1u, n16 = in & 15u;
+    uint32_t tn;
+    const uint32_t rb = div_by(u, a.nt, a.nt_inv, tn);
+    const uint32_t m = 16 * rb + n16;
+    const uint32_t n = T5_BN * tn + 64 * (wc >> 2) + 16 * (wc & 3u) + 8 * j;
+    const bool valid = u < a.units && m < a.M && n < a.N;
+    const size_t o = (size_t)m * a.N + n;
+    half_t bv[8], rv[8];
+    if (valid && part == 0) {
+        load_epi<8>(a.bias ? a.bias + n : nullptr, bv);
+        load_epi<8>(a.residual ? a.residual + o : nullptr, rv);
+    }
+    // A unit is 16 KB, a fragment 1 KB, lane 32 j + n16's value 16 bytes; all
+    // splits together are below 2^31 bytes.
+    const uint32_t step = a.units * 16384u, base = u * 16384u + wc * 1024u + (32 * j + n16) * 16u;
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.partials, a.split_k * step);
     floatx4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-    if (valid) {
-        // In float4: a unit is 1024, a fragment 64, lane 32 j + n16.
-        const floatx4* p = reinterpret_cast<const floatx4*>(partials) + (size_t)u * 1024 + 64 * wc + 32 * j + n16;
-        const size_t step = (size_t)RB * NT * 1024;  // one split
-#pragma unroll 4
-        for (int sp = part; sp < split_k; sp += P) {
-            sa += __builtin_nontemporal_load(p + (size_t)sp * step);
-            sb += __builtin_nontemporal_load(p + (size_t)sp * step + 16);
+    for (uint32_t s0 = part; s0 < a.split_k; s0 += U * P) {
+        u32x4 va[U], vb[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const uint32_t sp = s0 + i * P;
+            const uint32_t off = valid && sp < a.split_k ? sp * step + base : 0x80000000u;
+            va[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, off, 0u, kCpolNT));
+            vb[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, off + 256u, 0u, kCpolNT));
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            sa += __builtin_bit_cast(floatx4, va[i]);
+            sb += __builtin_bit_cast(floatx4, vb[i]);
         }
     }
-    fin[0][t] = sa;
-    fin[1][t] = sb;
-    __syncthreads();
+    if constexpr (P > 1) {
+        fin[0][t] = sa;
+        fin[1][t] = sb;
+        __syncthreads();
+    }
     if (valid && part == 0) {
+#pragma unroll
         for (int i = 1; i < P; ++i) {
-            sa += fin[0][i * per_wg + t];
-            sb += fin[1][i * per_wg + t];
+            sa += fin[0][i * kPieces + t];
+            sb += fin[1][i * kPieces + t];
         }
         const float y[8] = {sa[0], sb[0], sa[1], sb[1], sa[2], sb[2], sa[3], sb[3]};
-        store_out<8>(out, bias, residual, N, m, n, y);
+        half8_t h;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) h[i] = epi_round_vals(y[i], a.bias != nullptr, bv[i], a.residual != nullptr, rv[i]);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, h), make_rsrc(a.out, 0x7FFFFFFFu),
+                                               (uint32_t)(o * 2), 0, kCpolSC1);
     }
 }
 
@@ -737,9 +771,14 @@ hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* count
         }
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess || !reduce || cfg.split_k <= 1) return e;
-        hipLaunchKernelGGL(awq_tile_reduce_kernel, dim3((unsigned)tile_reduce_blocks(a.M, a.N, cfg.split_k)), dim3(256),
-                           0, stream, a.partials, a.out, a.bias, a.residual, a.M, a.N, cfg.split_k,
-                           stream_reduce_parts(cfg.split_k));
+        const uint32_t nt = (uint32_t)((a.N + T5_BN - 1) / T5_BN);
+        const TileReduceArgs r{a.partials, a.out, a.bias, a.residual, (uint32_t)a.M, (uint32_t)a.N,
+                               (uint32_t)cfg.split_k, nt, div_inverse(nt), (uint32_t)((a.M + 15) / 16) * nt};
+        const dim3 rgrid((unsigned)tile_reduce_blocks(a.M, a.N, cfg.split_k));
+        with_reduce_shape(cfg.split_k, [&](auto parts, auto unroll) {
+            hipLaunchKernelGGL((awq_tile_reduce_kernel<decltype(parts)::value, decltype(unroll)::value>), rgrid,
+                               dim3(256), 0, stream, r);
+        });
         return hipGetLastError();
     }
     return hipErrorInvalidValue;
