@@ -211,6 +211,13 @@ __device__ __forceinline__ void wait_batches(int n) {
     }
 }
 
+// SiLU(x) * u in fp32 (kernels/silu_mul.py:17-39: x * sigmoid(x) * y).  The
+// hardware reciprocal (1 ulp) where a correctly rounded division takes ten
+// instructions more.
+__device__ __forceinline__ float silu_mul(float x, float u) {
+    return x * __builtin_amdgcn_rcpf(1.0f + expf(-x)) * u;
+}
+
 // Division by a kernel argument whose reciprocal the host passes: n / d and
 // the remainder for n < 2^31, inv = div_inverse(d) = ceil(2^31 / d).  inv
 // exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less

@@ -494,10 +494,7 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(QuadArgs a) {
             half8_t v = __builtin_bit_cast(half8_t, xv[i]);
             const half8_t u = __builtin_bit_cast(half8_t, xw[i]);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float x = (float)v[e];
-                v[e] = (half_t)(x / (1.0f + expf(-x)) * (float)u[e]);
-            }
+            for (int e = 0; e < 8; ++e) v[e] = (half_t)silu_mul((float)v[e], (float)u[e]);
             xv[i] = __builtin_bit_cast(u32x4, v);
         }
     }
