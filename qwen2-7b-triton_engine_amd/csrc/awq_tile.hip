@@ -107,10 +107,24 @@ __device__ __forceinline__ int hy_bands(int n_sk, int d, int bm) {
 // 256-column tiles, two workgroups per CU for 128 rows; 8: 512-column tiles,
 // one workgroup per CU, FIN 1 and no hybrid only -- variant 15).  The x rows
 // of a k-step are loaded once for all of the workgroup's columns.
+//
+// The arguments that place a workgroup are read with one wait, and its tile
+// is found without an integer division by an argument (TileGeom): before
+// that a workgroup ran some 300 instructions and three serial argument loads
+// ahead of its first load.  0.15 - 0.2 us a call: 3584 x 3584 at M = 16 9.0 ->
+// 8.8 us, at M = 700 31.95 -> 31.7; the same at M = 2048.
+struct TileGeom {
+    uint32_t total;                            // workgroups
+    uint32_t split_inv, tiles_inv, group_inv;  // div_inverse of split_k, of the tiles, of T5_GM rows of tiles
+};
 template <int FM, int FIN, bool HY = false, int NW = 4>
 __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_kernel(GemmArgs a, int split_k,
                                                                               int k_per_split,
-                                                                              uint32_t* counters) {
+                                                                              uint32_t* counters, TileGeom geo) {
+    if constexpr (!HY)
+        asm volatile("" ::"s"(a.x), "s"(a.qweight), "s"(a.qzeros), "s"(a.scales), "s"(a.M), "s"(a.N), "s"(a.K),
+                     "s"(split_k), "s"(k_per_split), "s"(geo.total), "s"(geo.split_inv), "s"(geo.tiles_inv),
+                     "s"(geo.group_inv));
     using L = T5Layout<FM, NW>;
     constexpr int BN = L::BN;
     constexpr int BM = L::BM;
@@ -132,25 +146,25 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
     const int kb = lane >> 4;
 
     // ---- work item: XCD-aware grouped tile order (groups of T5_GM row tiles) ----
-    const int m_tiles = (a.M + BM - 1) / BM;
-    const int n_tiles = (a.N + BN - 1) / BN;
+    const int m_tiles = (int)((uint32_t)(a.M + BM - 1) / (uint32_t)BM);
+    const int n_tiles = (int)((uint32_t)(a.N + BN - 1) / (uint32_t)BN);
+    uint32_t rem;
     // Position of workgroup b among `total` consecutive ones in XCD order:
     // the workgroups one XCD runs (b % 8 == x) get consecutive positions.
     auto xcd_order = [](int b, int total) {
-        const int xcd = b & 7, xi = b >> 3, per = (total + 7) >> 3, rem = total & 7;
-        return (rem == 0 || xcd < rem) ? xcd * per + xi : rem * per + (xcd - rem) * (per - 1) + xi;
+        return (b & 7) * (total >> 3) + min(b & 7, total & 7) + (b >> 3);
     };
     int tile, split, ks = split_k, sk_tile = 0, n_sk = 0;  // ks: splits of this workgroup's tile
     if constexpr (HY) {
         const int T = m_tiles * n_tiles;
-        n_sk = ((int)gridDim.x - T) / (split_k - 1);
+        n_sk = ((int)geo.total - T) / (split_k - 1);
         const int D = T - n_sk;
         if ((int)blockIdx.x < D) {
             tile = xcd_order((int)blockIdx.x, D);
             split = 0;
             ks = 1;
         } else {
-            const int w = xcd_order((int)blockIdx.x - D, (int)gridDim.x - D);
+            const int w = xcd_order((int)blockIdx.x - D, (int)geo.total - D);
             sk_tile = w / split_k;
             tile = D + sk_tile;
             split = w - sk_tile * split_k;
@@ -164,22 +178,32 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
         // outputs are the same in either order.  Measured 1 - 3 % faster on
         // K = 18944 (down_proj) at M = 96 - 2048, and 2 - 3 % slower on K =
         // 3584, hence the bound.
-        const int T = m_tiles * n_tiles;
-        const int w = xcd_order((int)blockIdx.x, (int)gridDim.x);
-        split = w / T;
-        tile = w - split * T;
+        const uint32_t w = (uint32_t)xcd_order((int)blockIdx.x, (int)geo.total);
+        split = (int)div_by(w, (uint32_t)(m_tiles * n_tiles), geo.tiles_inv, rem);
+        tile = (int)rem;
     } else {
-        const int w = xcd_order((int)blockIdx.x, (int)gridDim.x);
-        tile = w / split_k;
-        split = w - tile * split_k;
+        const uint32_t w = (uint32_t)xcd_order((int)blockIdx.x, (int)geo.total);
+        tile = (int)div_by(w, (uint32_t)split_k, geo.split_inv, rem);
+        split = (int)rem;
     }
     const int in_group = T5_GM * n_tiles;
     // Tile t's first row and column (tiles in groups of T5_GM row tiles).
     auto tile_origin = [&](int t, int& tm0, int& tn0) {
-        const int first_m = (t / in_group) * T5_GM;
+        if constexpr (HY) {  // called again at the end: plain divisions keep nothing in registers until then
+            const int first_m = (t / in_group) * T5_GM;
+            const int gm = min(m_tiles - first_m, T5_GM);
+            tm0 = (first_m + (t % in_group) % gm) * BM;
+            tn0 = ((t % in_group) / gm) * BN;
+            return;
+        }
+        uint32_t in, row;
+        const int first_m = (int)div_by((uint32_t)t, (uint32_t)in_group, geo.group_inv, in) * T5_GM;
         const int gm = min(m_tiles - first_m, T5_GM);
-        tm0 = (first_m + (t % in_group) % gm) * BM;
-        tn0 = ((t % in_group) / gm) * BN;
+        static_assert(T5_GM == 4, "the inverses of 1 .. 4");
+        const uint32_t inv = gm == 4 ? 0x20000000u : gm == 3 ? 0x2AAAAAABu : gm == 2 ? 0x40000000u : 0x80000000u;
+        const uint32_t column = div_by(in, (uint32_t)gm, inv, row);
+        tm0 = (first_m + (int)row) * BM;
+        tn0 = (int)column * BN;
     };
     int m0, n0;
     tile_origin(tile, m0, n0);
@@ -563,7 +587,7 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
         if constexpr (HY) {
             // Whole-tile workgroup b < n_sk * H helps finish band b % H of
             // leftover tile b / H (below).
-            const int hb = hy_bands(n_sk, (int)gridDim.x - n_sk * split_k, BM);
+            const int hb = hy_bands(n_sk, (int)geo.total - n_sk * split_k, BM);
             if ((int)blockIdx.x < n_sk * hb) {
                 __syncthreads();  // the staged tile's reads are done: the LDS becomes `fin`
                 if (tid == 0)
@@ -607,7 +631,7 @@ __global__ __launch_bounds__(64 * NW, (T5Layout<FM, NW>::PER_CU)) void awq_tile_
         // own tile) each add 1 to; whoever brings it to split_k + 1 adds the
         // band's partials.  The helpers run late, so usually they do, spread
         // over many workgroups instead of one last piece per tile.
-        const int hb = hy_bands(n_sk, (int)gridDim.x - n_sk * split_k, BM);
+        const int hb = hy_bands(n_sk, (int)geo.total - n_sk * split_k, BM);
         if (tid < hb)
             last_band[tid] = __hip_atomic_fetch_add(&counters[sk_tile * hb + tid], 1u, __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)split_k;
@@ -725,10 +749,15 @@ int64_t tile_tiles(int M, int N, int variant) {
     return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 
-// The reduce-finish tile with FM 16-row blocks of x.
-template <int FM>
+// FM 16-row blocks of x per tile.
+template <int FM, int FIN = 1, bool HY = false, int NW = 4>
 static void tile_launch(const GemmArgs& a, const TileConfig& cfg, dim3 grid, uint32_t* counters, hipStream_t stream) {
-    hipLaunchKernelGGL((awq_tile_kernel<FM, 1>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters);
+    using L = T5Layout<FM, NW>;
+    const uint32_t n_tiles = (uint32_t)((a.N + L::BN - 1) / L::BN), m_tiles = (uint32_t)((a.M + L::BM - 1) / L::BM);
+    const TileGeom geo{grid.x, div_inverse((uint32_t)cfg.split_k), div_inverse(m_tiles * n_tiles),
+                       div_inverse(T5_GM * n_tiles)};
+    hipLaunchKernelGGL((awq_tile_kernel<FM, FIN, HY, NW>), grid, dim3(64 * NW), 0, stream, a, cfg.split_k,
+                       cfg.k_per_split, counters, geo);
 }
 
 hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* counters, hipStream_t stream) {
@@ -738,7 +767,7 @@ hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* count
         const dim3 grid((unsigned)blocks);
         bool reduce = false;
         switch (cfg.variant) {
-            case 6: hipLaunchKernelGGL((awq_tile_kernel<8, 0>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
+            case 6: tile_launch<8, 0>(a, cfg, grid, counters, stream); break;
             case 7:
             case 8:
             case 9: {
@@ -764,9 +793,9 @@ hipError_t launch_tile(const GemmArgs& a, const TileConfig& cfg, uint32_t* count
                 }
                 break;
             }
-            case 15: hipLaunchKernelGGL((awq_tile_kernel<8, 1, false, 8>), grid, dim3(512), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); reduce = true; break;
-            case 13: hipLaunchKernelGGL((awq_tile_kernel<8, 0, true>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
-            case 14: hipLaunchKernelGGL((awq_tile_kernel<4, 0, true>), grid, dim3(256), 0, stream, a, cfg.split_k, cfg.k_per_split, counters); break;
+            case 15: tile_launch<8, 1, false, 8>(a, cfg, grid, counters, stream); reduce = true; break;
+            case 13: tile_launch<8, 0, true>(a, cfg, grid, counters, stream); break;
+            case 14: tile_launch<4, 0, true>(a, cfg, grid, counters, stream); break;
             default: return hipErrorInvalidValue;
         }
         const hipError_t e = hipGetLastError();
