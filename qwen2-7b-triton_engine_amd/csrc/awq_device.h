@@ -218,6 +218,27 @@ __device__ __forceinline__ float silu_mul(float x, float u) {
     return x * __builtin_amdgcn_rcpf(1.0f + expf(-x)) * u;
 }
 
+// Sum over a wave, the same in every lane: DPP steps within the rows of 16
+// lanes, then the four rows' sums.  (Six ds_bpermute steps wait for the LDS
+// pipe six times.)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dpp_move<0x141>(v);  // row_half_mirror
+    v += dpp_move<0x140>(v);  // row_mirror
+    const int i = __builtin_bit_cast(int, v);
+    auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, lane)); };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
+// RMSNorm's factor 1 / sqrt(sum / H + eps), inv_h = 1 / H (v_rsq_f32: 1 ulp).
+__device__ __forceinline__ float norm_factor(float sum, float inv_h, float eps) {
+    return __builtin_amdgcn_rsqf(__builtin_fmaf(sum, inv_h, eps));
+}
+
 // Division by a kernel argument whose reciprocal the host passes: n / d and
 // the remainder for n < 2^31, inv = div_inverse(d) = ceil(2^31 / d).  inv
 // exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less

@@ -245,9 +245,10 @@ __global__ __launch_bounds__(512) void awq_gemv_stream_kernel(GemmArgs a, int ch
 // takes the RMSNorm of the row (every workgroup sums the whole row's squares,
 // 7 KB from L2, and scales its own K range), kInputSiluMul takes SiLU(gate) *
 // up of its K range.  A launch in a replayed graph costs 2.1 us however small;
-// measured in graphs over 28 layers' weights, us, fused / two launches: norm
-// + 3584 x 4608 6.3 / 7.7, norm + 3584 x 37888 17.3 / 18.6, SiLU * up + 18944 x
-// 3584 11.3 / 13.1; a decoder layer 53.7 / 57.7 (50 with the short lead below).
+// measured in graphs over 28 layers' weights, us, fused / two launches / the
+// projection alone: norm + 3584 x 4608 5.1 / 6.6 / 4.7, norm + 3584 x 37888
+// 16.7 / 17.9 / 16.0, SiLU * up + 18944 x 3584 10.5 / 12.5 / 10.2; a decoder
+// layer 46.7 / 52.5.
 //
 // The way to the first load.  At 5 us a call, the time before a workgroup's
 // first weight load counts: every kernel argument line is a cold scalar load,
@@ -279,7 +280,7 @@ struct QuadArgs {
     unsigned long long* fix;
     float* partials;
     const half_t* norm_w;            // kInputNorm
-    float norm_eps;
+    float norm_eps, norm_inv_k;
 };
 static_assert(offsetof(QuadArgs, out) == 64 && sizeof(QuadArgs) <= 128, "two lines");
 
@@ -472,13 +473,14 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(QuadArgs a) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)v[e], (float)v[e], s);
         }
-#pragma unroll
-        for (int w = 1; w < 64; w *= 2) s += __shfl_xor(s, w);
-        if (lane == 0) squares[wave] = s;
+        s = wave_sum(s);
+        // Wave 0 also clears the places of waves that the workgroup does not have.
+        if (wave == 0 ? lane == 0 || (lane >= nw && lane < 8) : lane == 0) squares[wave + lane] = lane == 0 ? s : 0.f;
         __syncthreads();
         s = 0.f;
-        for (int w = 0; w < nw; ++w) s += squares[w];
-        const float r = 1.0f / sqrtf(s / (float)a.K + a.norm_eps);
+#pragma unroll
+        for (int w = 0; w < 8; ++w) s += squares[w];
+        const float r = norm_factor(s, a.norm_inv_k, a.norm_eps);
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             half8_t v = __builtin_bit_cast(half8_t, xv[i]);
@@ -688,6 +690,7 @@ static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uin
     q.partials = a.partials;
     q.norm_w = cfg.norm_w;
     q.norm_eps = cfg.norm_eps;
+    q.norm_inv_k = 1.0f / (float)a.K;
     q.total = grid.x;
     // Weight loads marked non-temporal where each workgroup streams a long
     // K range (few splits): 3584 x 37888 at split 3 measured 2.7 - 4.7 %

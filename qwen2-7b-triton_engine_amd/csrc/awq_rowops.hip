@@ -6,12 +6,6 @@ namespace {
 
 constexpr int kNormThreads = 512;
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int w = 1; w < 64; w *= 2) v += __shfl_xor(v, w);
-    return v;
-}
-
 // out[m] = fp16(x[m] * rsqrt(mean(x[m]^2) + eps) * w) in fp32
 // (model/qwen2.py:15-22).  One workgroup per row, C 16-byte pieces of it per
 // thread held in registers between the sum and the store: the row is read
@@ -23,7 +17,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 template <int C>
 __global__ __launch_bounds__(kNormThreads) void awq_rmsnorm_kernel(const half_t* __restrict__ x,
                                                                    const half_t* __restrict__ w,
-                                                                   half_t* __restrict__ out, int H, float eps) {
+                                                                   half_t* __restrict__ out, int H, float inv_h,
+                                                                   float eps) {
     __shared__ float sums[kNormThreads / 64];
     const int pieces = H / 8;
     const half8_t* xr = reinterpret_cast<const half8_t*>(x + (size_t)blockIdx.x * H);
@@ -50,7 +45,7 @@ __global__ __launch_bounds__(kNormThreads) void awq_rmsnorm_kernel(const half_t*
     s = 0.0f;
 #pragma unroll
     for (int i = 0; i < kNormThreads / 64; ++i) s += sums[i];
-    const float r = 1.0f / sqrtf(s / (float)H + eps);
+    const float r = norm_factor(s, inv_h, eps);
     half8_t* orow = reinterpret_cast<half8_t*>(out + (size_t)blockIdx.x * H);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -71,7 +66,7 @@ hipError_t launch_rmsnorm(const half_t* x, const half_t* w, half_t* out, int M, 
     if (M == 0) return hipSuccess;
     const int c = (H / 8 + kNormThreads - 1) / kNormThreads;
     auto kernel = c <= 1 ? awq_rmsnorm_kernel<1> : c <= 2 ? awq_rmsnorm_kernel<2> : awq_rmsnorm_kernel<4>;
-    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, H, eps);
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, H, 1.0f / (float)H, eps);
     return hipGetLastError();
 }
 
