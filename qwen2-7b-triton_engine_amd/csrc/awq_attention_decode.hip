@@ -11,8 +11,8 @@
 // enough workgroups to load it at once, each keeps a running softmax of its
 // range for all query heads of one KV head (so K and V are read once), and a
 // second launch weights the ranges' partial sums.  Measured on Qwen2-7B's
-// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 8.8 us for
-// the two at position 1100, where two empty launches take 4.2; 10.2 with eight
+// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 8.4 us for
+// the two at position 1100, where two small launches take 4; 10.2 with eight
 // waves a workgroup (two per SIMD: the kernel is then bound by its own
 // instructions) and its loads behind the position's; 17 with the scores, the
 // softmax and P V on the vector unit, 16 lanes a key.
@@ -252,7 +252,8 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
                                                                     int chunk, int ranges) {
     __shared__ float o_lds[4][HD];
     const int64_t pos = *posp;
-    const int head = blockIdx.x, d = threadIdx.x % HD, quarter = threadIdx.x / HD, lane = threadIdx.x & 63;
+    const int head = blockIdx.x, d = threadIdx.x % HD, lane = threadIdx.x & 63;
+    const int quarter = __builtin_amdgcn_readfirstlane(threadIdx.x / HD);   // the same for a wave
     const size_t step = (size_t)nh * (HD + 2);
     const float* base = part + (size_t)head * (HD + 2);
     // Loaded before the position is known; what no range wrote this time is
@@ -269,13 +270,9 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
         mine = -INFINITY;
         l = 0.0f;
     }
-    float mx = mine;
-#pragma unroll
-    for (int w = 1; w < 64; w *= 2) mx = fmaxf(mx, __shfl_xor(mx, w));
+    const float mx = wave_max(mine);
     const float a = __builtin_amdgcn_exp2f(mine - (mx == -INFINITY ? 0.0f : mx));
-    l *= a;
-#pragma unroll
-    for (int w = 1; w < 64; w *= 2) l += __shfl_xor(l, w);
+    l = wave_sum(l * a);
     float sum = 0.0f;
     for (int i0 = quarter; i0 < n; i0 += 32) {
         if (i0 != quarter) {
@@ -284,7 +281,8 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float w = __shfl(a, (i0 + 4 * j) & 63);
+            const float w = __builtin_bit_cast(
+                float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), (i0 + 4 * j) & 63));
             sum = fmaf(w, i0 + 4 * j < n ? v[j] : 0.0f, sum);
         }
     }

@@ -234,6 +234,16 @@ __device__ __forceinline__ float wave_sum(float v) {
     auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, lane)); };
     return (row(0) + row(16)) + (row(32) + row(48));
 }
+// Maximum over a wave, the same in every lane.
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, dpp_move<0xB1>(v));
+    v = fmaxf(v, dpp_move<0x4E>(v));
+    v = fmaxf(v, dpp_move<0x141>(v));
+    v = fmaxf(v, dpp_move<0x140>(v));
+    const int i = __builtin_bit_cast(int, v);
+    auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, lane)); };
+    return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
+}
 // RMSNorm's factor 1 / sqrt(sum / H + eps), inv_h = 1 / H (v_rsq_f32: 1 ulp).
 __device__ __forceinline__ float norm_factor(float sum, float inv_h, float eps) {
     return __builtin_amdgcn_rsqf(__builtin_fmaf(sum, inv_h, eps));
