@@ -13,6 +13,12 @@
 // the Python mirror's (kernels/awq_gemm.py in this package): ValueError for
 // a bad operand, RuntimeError for a failed launch.
 //
+// gemm is the same with the bias and residual adds (awq_gemm_forward_ex's AUTO
+// path), qwen2_layer a whole decoder layer of the engine.  At M = 1 a kernel
+// takes 5 - 17 us and a call through ctypes 10: 16 layers' projections issued
+// eagerly took 612 us, 579 through here; eight eager decode steps of four
+// layers 3.85 ms, 3.02.
+//
 // Workspace registry: one list of zero-filled float32 buffers per device,
 // grown on demand and never shrunk; earlier buffers stay referenced so that
 // graphs captured with them keep valid memory.  Counters and fixed-point
