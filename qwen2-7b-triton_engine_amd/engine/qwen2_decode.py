@@ -29,6 +29,7 @@ from __future__ import annotations
 
 import dataclasses
 import math
+import operator
 import time
 
 import torch
@@ -254,6 +255,7 @@ class Qwen2AwqDecoder:
     @torch.no_grad()
     def decode_logits(self, token: torch.Tensor, pos: int) -> torch.Tensor:
         """One eager decode step: logits after feeding `token` at position `pos`."""
+        pos = operator.index(pos)
         if not 0 <= pos < self.max_seq_len:
             raise ValueError(f"position {pos} outside [0, {self.max_seq_len})")
         # filled on the device: a tensor made from host data would wait for the stream

@@ -69,3 +69,4 @@ def test_positions_outside_the_cache_are_refused(gpu):
     with pytest.raises(ValueError):
         m.prefill(torch.zeros(9, dtype=torch.int64))
     m.prefill(torch.zeros(8, dtype=torch.int64))
+    assert torch.equal(m.decode_logits(torch.tensor(3), torch.tensor(7)), m.decode_logits(torch.tensor(3), 7))
