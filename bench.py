@@ -901,8 +901,8 @@ def main():
             "prefill_ms": round(r["prefill_s"] * 1e3, 2),
             "decode_ms_per_token": round(r["decode_s"] / 127 * 1e3, 3),
             "decode_tokens_per_s": round(r["decode_tokens_per_s"], 1),
-            "note": "greedy, batch 1, one HIP graph replay per token; AWQ linears and lm_head on this "
-                    "build's kernels, the other ops torch",
+            "note": "greedy, batch 1, one HIP graph replay per token; projections, norms, attention and "
+                    "lm_head on the HIP kernels, embedding and the greedy choice in torch",
         }
         del e2e
         torch.cuda.empty_cache()
