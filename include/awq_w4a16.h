@@ -368,7 +368,7 @@ int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, con
  * with rows 0 .. S - 1 of the caches written.  qkv fp16 [S, (num_heads + 2
  * num_kv_heads) * head_dim], out fp16 [S, num_heads * head_dim], S <= max_seq;
  * S == 0 is a valid no-op.  q and the probabilities enter the matrix cores as
- * sums of two fp16 values (22 bits), with fp32 sums.  workspace: at least
+ * sums of two fp16 values (23 bits), with fp32 sums.  workspace: at least
  * awq_fp16_attention_prefill_workspace bytes, of any content; it holds nothing
  * between calls.  Two launches. */
 size_t awq_fp16_attention_prefill_workspace(int64_t S, int64_t num_kv_heads, int64_t head_dim);

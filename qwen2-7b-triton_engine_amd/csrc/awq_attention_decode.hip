@@ -25,23 +25,7 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kHeads = 16;             // query heads of one workgroup: the columns of an MFMA
 constexpr int kKeys = 16 * kWaves;     // positions of one inner pass of a workgroup: 16 per wave
-constexpr float kQScale = 4.0f;        // see split16
 constexpr float kPExp = 14.0f;
-
-// x = hi + lo in two fp16 values, 22 bits while lo stays above fp16's
-// smallest steps: q is scaled by 4 and the probabilities by 2^14 before the
-// split, powers of two that cancel exactly.  x is made opaque first: the
-// compiler would otherwise round the product that x is straight to fp16 for
-// one use of hi and by way of fp32 for the other.
-template <int N, typename V>
-__device__ __forceinline__ void split16(float (&x)[N], V& hi, V& lo) {
-#pragma unroll
-    for (int e = 0; e < N; ++e) {
-        asm("" : "+v"(x[e]));
-        hi[e] = (half_t)x[e];
-        lo[e] = (half_t)(x[e] - (float)hi[e]);
-    }
-}
 
 // One workgroup: positions [split * chunk, ...) of one KV head for up to 16
 // query heads, 16 positions per wave and pass.  S^T = K Q^T on the MFMA: its
@@ -50,7 +34,7 @@ __device__ __forceinline__ void split16(float (&x)[N], V& hi, V& lo) {
 // V's row order in that product is free, so lane i takes columns i VC ..
 // i VC + VC - 1 of a V row with one load and supplies one of them to each of
 // VC products.  q and the probabilities are fp32 values split in two fp16
-// parts.  K, V and q are loaded before the position is known (rows of the
+// parts, q scaled by its head's largest value and the probabilities by 2^14.  K, V and q are loaded before the position is known (rows of the
 // cache past it are masked), so the chain is two memory latencies long: the
 // position, then the RoPE row it selects.  The waves' results meet once, at
 // the end.
@@ -121,23 +105,29 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
     __builtin_amdgcn_sched_barrier(0);   // every load above is issued before the first is waited for
 
     // RoPE of this lane's columns 32 st + 8 t .. + 7 of its head, and of the
-    // new key; exp(x / sqrt(HD) - max) = exp2((x - max) log2(e) / sqrt(HD)).
-    const float scale = kQScale * 1.4426950408889634f / sqrtf((float)HD);
+    // new key.
     const bool has_new = start <= pos && end == pos + 1;
     half8_t qhi[kSteps], qlo[kSteps], kn[kSteps] = {};
+    float x[kSteps][8], qmax = 0.0f;
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
         const bool low = st < kSteps / 2;
         const int other = low ? st + kSteps / 2 : st - kSteps / 2;
-        float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float cc = cs[st][e / 4][e % 4], ss = low ? -sn[st][e / 4][e % 4] : sn[st][e / 4][e % 4];
-            x[e] = ((float)qraw[st][e] * cc + (float)qraw[other][e] * ss) * scale;
+            x[st][e] = (float)qraw[st][e] * cc + (float)qraw[other][e] * ss;
+            qmax = fmaxf(qmax, fabsf(x[st][e]));
             if (has_new) kn[st][e] = (half_t)((float)kraw[st][e] * cc + (float)kraw[other][e] * ss);
         }
-        split16(x, qhi[st], qlo[st]);
     }
+    qmax = fmaxf(qmax, __shfl_xor(qmax, 16));
+    qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+    const int exp = split16_exp(qmax);
+    // exp(x / sqrt(HD)) = exp2(x c) = exp2(score unit), the scores being scaled like q
+    const float c = 1.4426950408889634f / sqrtf((float)HD), unit = __builtin_ldexpf(c, -exp);
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) split16(x[st], exp, qhi[st], qlo[st]);
     if (valid && has_new && blockIdx.z == 0 && wave == 0) {   // the caches' new row
         if (col == 0) {
 #pragma unroll
@@ -180,18 +170,18 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const float mn = fmaxf(m, mx);
-        const float ref = mn == -INFINITY ? 0.0f : mn / kQScale;   // nothing yet: every exponential is 0
-        const float alpha = __builtin_amdgcn_exp2f(m / kQScale - ref);
+        const float ref = mn == -INFINITY ? 0.0f : mn * unit;   // nothing yet: every exponential is 0
+        const float alpha = __builtin_amdgcn_exp2f(fmaf(m, unit, -ref));
         m = mn;
         float p[4];
         l *= alpha;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], 1.0f / kQScale, kPExp - ref));
+            p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], unit, kPExp - ref));
             l += p[r];
         }
         half4_t phi, plo;
-        split16(p, phi, plo);
+        split16(p, 0, phi, plo);
 #pragma unroll
         for (int v = 0; v < VC; ++v) {
             const half4_t a = {vf[0][v], vf[1][v], vf[2][v], vf[3][v]};
@@ -206,7 +196,7 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
     // This lane: rows 4 t + r of each product, i.e. columns VC (4 t + r) + v of head `col`.
     if (col < heads) {
         if (t == 0) {
-            m_lds[wave][col] = m;
+            m_lds[wave][col] = __builtin_ldexpf(m, -exp);   // of the scores themselves
             l_lds[wave][col] = l;
         }
 #pragma unroll
@@ -228,14 +218,14 @@ __global__ __launch_bounds__(kThreads) void awq_decode_attn_kernel(
         float sum = 0.0f, ls = 0.0f;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const float a = __builtin_amdgcn_exp2f((m_lds[w][h] - ref) / kQScale);
+            const float a = __builtin_amdgcn_exp2f((m_lds[w][h] - ref) * c);
             sum = fmaf(a, o_lds[w][h][d], sum);
             ls = fmaf(a, l_lds[w][h], ls);
         }
         float* dst = part + ((size_t)split * nh + g * groups + h0 + h) * (HD + 2);
         dst[d] = sum;
         if (d == 0) {
-            dst[HD] = mx / kQScale;
+            dst[HD] = mx * c;
             dst[HD + 1] = ls;
         }
     }

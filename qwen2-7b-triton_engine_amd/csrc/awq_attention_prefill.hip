@@ -14,11 +14,12 @@
 // Precision.  K and V are fp16 in the cache; q after RoPE and the
 // probabilities are fp32 and stay so: each is split into two fp16 parts, hi =
 // fp16(x) and lo = fp16(x - hi), and both go through the fp16 MFMA with its
-// fp32 sums.  hi + lo carries 22 bits while lo is above fp16's smallest
-// steps (2^-24), so both operands are scaled up first: q by 4 (|q| <= 65504
-// sqrt(2) from fp16, times 4 log2(e) / sqrt(64), stays finite), the
-// probabilities, at most 1, by 2^14.  Scales are powers of two and cancel
-// exactly.
+// fp32 sums.  hi + lo carries 23 bits while lo is above fp16's smallest
+// steps (2^-24), so both operands are scaled first: a query row by the power
+// of two that brings its largest value to 2^14 .. 2^15 (RoPE makes up to 65504
+// sqrt(2) of fp16 values, more than fp16 holds), the probabilities, at most
+// 1, by 2^14.  Such scales cancel exactly.  log2(e) / sqrt(HD) is no power of
+// two and multiplies the scores, in fp32.
 #include "awq_kernels.h"
 
 namespace awq {
@@ -27,7 +28,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kKeys = 64;           // keys per tile
-constexpr float kQScale = 4.0f;
 constexpr float kPExp = 14.0f;
 
 // Position of a key within its 64-key tile of the transposed V: the S^T
@@ -99,18 +99,6 @@ __global__ __launch_bounds__(kThreads) void awq_prefill_kv_kernel(const half_t* 
     }
 }
 
-// x is made opaque first: the compiler would otherwise round the product that
-// x is once straight to fp16 for one use of hi and by way of fp32 for the
-// other, and where the two differ lo belongs to the wrong hi.
-__device__ __forceinline__ void split16(float (&x)[8], half8_t& hi, half8_t& lo) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        asm("" : "+v"(x[e]));
-        hi[e] = (half_t)x[e];
-        lo[e] = (half_t)(x[e] - (float)hi[e]);
-    }
-}
-
 // One workgroup: 64 NQ queries of one head, 16 NQ per wave, over the 64-key
 // tiles up to its last query.  S^T = K Q^T puts a query in each MFMA column,
 // so a query's running maximum and sum are one value per lane column, and the
@@ -164,8 +152,8 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
     issue(0, 0);
 
     half8_t qhi[NQ][kSteps], qlo[NQ][kSteps];
+    float unit[NQ];            // exp(x / sqrt(HD)) = exp2(score * unit)
     {
-        const float scale = kQScale * 1.4426950408889634f / sqrtf((float)HD);
         const size_t ld = (size_t)(nh + 2 * kvh) * HD;
 #pragma unroll
         for (int n = 0; n < NQ; ++n) {
@@ -174,20 +162,26 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
             half8_t raw[kSteps];
 #pragma unroll
             for (int st = 0; st < kSteps; ++st) raw[st] = *reinterpret_cast<const half8_t*>(src + 32 * st);
+            float x[kSteps][8], mx = 0.0f;
 #pragma unroll
             for (int st = 0; st < kSteps; ++st) {
                 const bool low = st < kSteps / 2;
                 const half8_t b = raw[low ? st + kSteps / 2 : st - kSteps / 2];
                 const floatx4* c = reinterpret_cast<const floatx4*>(cosp + (size_t)q * HD + 32 * st + 8 * t);
                 const floatx4* s = reinterpret_cast<const floatx4*>(sinp + (size_t)q * HD + 32 * st + 8 * t);
-                float x[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float p = (float)b[e];
-                    x[e] = ((float)raw[st][e] * c[e / 4][e % 4] + (low ? -p : p) * s[e / 4][e % 4]) * scale;
+                    x[st][e] = (float)raw[st][e] * c[e / 4][e % 4] + (low ? -p : p) * s[e / 4][e % 4];
+                    mx = fmaxf(mx, fabsf(x[st][e]));
                 }
-                split16(x, qhi[n][st], qlo[n][st]);
             }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const int exp = split16_exp(mx);
+            unit[n] = __builtin_ldexpf(1.4426950408889634f / sqrtf((float)HD), -exp);
+#pragma unroll
+            for (int st = 0; st < kSteps; ++st) split16(x[st], exp, qhi[n][st], qlo[n][st]);
         }
     }
 
@@ -249,9 +243,9 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float mn = fmaxf(m[n], mx);
-            const float ref = mn == -INFINITY ? 0.0f : mn / kQScale;   // nothing yet: every exponential is 0
+            const float ref = mn == -INFINITY ? 0.0f : mn * unit[n];   // nothing yet: every exponential is 0
             if (__any(mn > m[n])) {
-                const float alpha = __builtin_amdgcn_exp2f(m[n] / kQScale - ref);
+                const float alpha = __builtin_amdgcn_exp2f(fmaf(m[n], unit[n], -ref));
                 l[n] *= alpha;
 #pragma unroll
                 for (int d = 0; d < kDb; ++d) acc[n][d] *= alpha;
@@ -262,10 +256,10 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
                 float p[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    p[j] = __builtin_amdgcn_exp2f(fmaf(s[n][2 * h + (j >> 2)][j & 3], 1.0f / kQScale, kPExp - ref));
+                    p[j] = __builtin_amdgcn_exp2f(fmaf(s[n][2 * h + (j >> 2)][j & 3], unit[n], kPExp - ref));
                     l[n] += p[j];
                 }
-                split16(p, phi[n][h], plo[n][h]);
+                split16(p, 0, phi[n][h], plo[n][h]);
             }
         }
 #pragma unroll

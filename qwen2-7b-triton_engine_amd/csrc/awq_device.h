@@ -249,6 +249,25 @@ __device__ __forceinline__ float norm_factor(float sum, float inv_h, float eps) 
     return __builtin_amdgcn_rsqf(__builtin_fmaf(sum, inv_h, eps));
 }
 
+// x 2^exp = hi + lo in two fp16 values, 23 bits of it while lo stays above
+// fp16's smallest steps (2^-24).  The product with a power of two is exact, so
+// the two uses of hi agree however the compiler forms them.
+template <int N, typename V>
+__device__ __forceinline__ void split16(const float (&x)[N], int exp, V& hi, V& lo) {
+    const float scale = __builtin_ldexpf(1.0f, exp);
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        hi[e] = (half_t)(x[e] * scale);
+        lo[e] = (half_t)__builtin_fmaf(x[e], scale, -(float)hi[e]);
+    }
+}
+// The exponent for a row whose largest magnitude is mx: brought to 2^14 ..
+// 2^15, the row neither overflows fp16 nor loses low bits, whatever its size.
+__device__ __forceinline__ int split16_exp(float mx) {
+    const int e = 15 - __builtin_amdgcn_frexp_expf(mx);
+    return e < 100 ? e : 100;
+}
+
 // Division by a kernel argument whose reciprocal the host passes: n / d and
 // the remainder for n < 2^31, inv = div_inverse(d) = ceil(2^31 / d).  inv
 // exceeds 2^31 / d by less than 1, so the estimate exceeds n / d by less

@@ -148,3 +148,28 @@ def test_attention_decode_refuses(gpu):
     with pytest.raises(_native.AwqNativeError):        # head counts that do not divide
         attention_decode(torch.zeros((1, 7 * 64), dtype=torch.float16, device=gpu), c, c.clone(), cos, sin, pos, 3)
     assert attention_served(28, 4, 128, 2048) and not attention_served(4, 2, 32, 64)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("size", [65504.0, 1.0, 2.0**-10])
+def test_attention_queries_of_any_size(gpu, hd, size):
+    """Queries at fp16's limit, which RoPE takes past it (both halves of a
+    rotated pair at 65504, a rotation of 45 degrees: 92636), and small ones
+    against keys as much larger.  Scores of about 1 throughout."""
+    nh, kvh, S = 4, 2, 70
+    cos = torch.full((S, hd), math.sqrt(0.5), device=gpu)
+    g = torch.Generator().manual_seed(hd)
+    sign = torch.where(torch.rand((S, nh + 2 * kvh, hd // 2), generator=g) < 0.5, -1.0, 1.0)
+    qkv = torch.cat((sign, -sign), -1) * size                  # rotated: sqrt(2) size in the lower half
+    qkv[:, nh:nh + kvh] = torch.randn((S, kvh, hd), generator=g) / size
+    qkv[:, nh + kvh:] = torch.randn((S, kvh, hd), generator=g)
+    qkv = qkv.reshape(S, -1).half()
+    kc = torch.zeros((kvh, S, hd), dtype=torch.float16, device=gpu)
+    vc = kc.clone()
+    print(f"attention queries hd={hd} size={size}", flush=True)
+    out = attention_prefill(qkv.to(gpu), kc, vc, cos, cos, nh)
+    heads, c = qkv.double().view(S, -1, hd), cos.double().cpu()
+    ref = _attend64(_rope64(heads[:, :nh], c, c), kc.double().cpu(), heads[:, nh + kvh:].transpose(0, 1), 0)
+    _close(out, ref, "prefill")
+    one = attention_decode(qkv[-1:].contiguous().to(gpu), kc, vc, cos, cos, torch.tensor([S - 1], device=gpu), nh)
+    _close(one, ref[-1:], "decode")
