@@ -348,8 +348,9 @@ int awq_fp16_rmsnorm(const void* x, const void* w, void* out, int64_t M, int64_t
 /* Attention of one new position over a static KV cache (the decode step of
  * model/qwen2.py:104-163): rotate-half RoPE of q and k (fp32), k (rounded to
  * fp16) and v stored at row *pos of the caches, softmax(q K^T / sqrt(head_dim))
- * V over positions 0 .. *pos in fp32, out fp16.  qkv fp16 [(num_heads + 2
- * num_kv_heads) * head_dim]; k_cache / v_cache fp16 [num_kv_heads, max_seq,
+ * V over positions 0 .. *pos, out fp16.  q and the probabilities enter the
+ * matrix cores as sums of two fp16 values (23 bits), with fp32 sums.  qkv fp16
+ * [(num_heads + 2 num_kv_heads) * head_dim]; k_cache / v_cache fp16 [num_kv_heads, max_seq,
  * head_dim]; cos / sin fp32 [max_seq, head_dim]; pos int64 [1] on the device
  * (outside 0 .. max_seq - 1 nothing is written); out fp16 [num_heads *
  * head_dim].  head_dim 64 or 128 (AWQ_ERR_PATH otherwise), num_heads a
@@ -367,8 +368,7 @@ int awq_fp16_attention_decode(const void* qkv, void* k_cache, void* v_cache, con
  * model/qwen2.py:104-163): as awq_fp16_attention_decode for every position,
  * with rows 0 .. S - 1 of the caches written.  qkv fp16 [S, (num_heads + 2
  * num_kv_heads) * head_dim], out fp16 [S, num_heads * head_dim], S <= max_seq;
- * S == 0 is a valid no-op.  q and the probabilities enter the matrix cores as
- * sums of two fp16 values (23 bits), with fp32 sums.  workspace: at least
+ * S == 0 is a valid no-op.  workspace: at least
  * awq_fp16_attention_prefill_workspace bytes, of any content; it holds nothing
  * between calls.  Two launches. */
 size_t awq_fp16_attention_prefill_workspace(int64_t S, int64_t num_kv_heads, int64_t head_dim);

@@ -19,7 +19,11 @@
 // of two that brings its largest value to 2^14 .. 2^15 (RoPE makes up to 65504
 // sqrt(2) of fp16 values, more than fp16 holds), the probabilities, at most
 // 1, by 2^14.  Such scales cancel exactly.  log2(e) / sqrt(HD) is no power of
-// two and multiplies the scores, in fp32.
+// two and multiplies the difference of a score and the maximum, in fp32: the
+// scores reach 3e10, where the product's own rounding would be thousands.
+// Outputs that land on another fp16 value than the 64-bit result's, per
+// thousand, here / in plain fp32 attention (28 heads of 128, S = 1777): 1.1 /
+// 1.9, 1.9 / 3.3, 4.3 / 7.0 for queries and keys of standard deviation 0.3, 1, 2.
 #include "awq_kernels.h"
 
 namespace awq {
@@ -28,7 +32,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kKeys = 64;           // keys per tile
-constexpr float kPExp = 14.0f;
+constexpr int kPExp = 14;           // the probabilities' scale before they are split: 2^14
 
 // Position of a key within its 64-key tile of the transposed V: the S^T
 // product leaves lane group t (lanes 16 t ..) with keys 4 t .. 4 t + 3 of each
@@ -243,9 +247,9 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
             mx = fmaxf(mx, __shfl_xor(mx, 16));
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float mn = fmaxf(m[n], mx);
-            const float ref = mn == -INFINITY ? 0.0f : mn * unit[n];   // nothing yet: every exponential is 0
+            const float ref = mn == -INFINITY ? 0.0f : mn;   // nothing yet: every exponential is 0
             if (__any(mn > m[n])) {
-                const float alpha = __builtin_amdgcn_exp2f(fmaf(m[n], unit[n], -ref));
+                const float alpha = __builtin_amdgcn_exp2f((m[n] - ref) * unit[n]);
                 l[n] *= alpha;
 #pragma unroll
                 for (int d = 0; d < kDb; ++d) acc[n][d] *= alpha;
@@ -256,10 +260,10 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
                 float p[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    p[j] = __builtin_amdgcn_exp2f(fmaf(s[n][2 * h + (j >> 2)][j & 3], unit[n], kPExp - ref));
+                    p[j] = __builtin_amdgcn_exp2f((s[n][2 * h + (j >> 2)][j & 3] - ref) * unit[n]);
                     l[n] += p[j];
                 }
-                split16(p, 0, phi[n][h], plo[n][h]);
+                split16(p, kPExp, phi[n][h], plo[n][h]);
             }
         }
 #pragma unroll
@@ -282,6 +286,7 @@ __global__ __launch_bounds__(kThreads, 2) void awq_prefill_attn_kernel(
         float sum = l[n];
         sum += __shfl_xor(sum, 16);
         sum += __shfl_xor(sum, 32);
+        sum = __builtin_ldexpf(sum, kPExp);
         const int q = q0 + 16 * n + col;
         if (q >= S) continue;
         half_t* dst = out + ((size_t)q * nh + head) * HD + 4 * t;

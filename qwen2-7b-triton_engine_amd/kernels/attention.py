@@ -2,9 +2,11 @@
 
 ``attention_decode`` is one new position over a static KV cache, from the
 fused QKV projection to the attention output: RoPE, the cache's new row,
-softmax(q K^T / sqrt(d)) V in fp32 (``model/qwen2.py:104-163``,
+softmax(q K^T / sqrt(d)) V (``model/qwen2.py:104-163``,
 ``kernels/rope.py:41-57``) -- two launches.  ``attention_prefill`` is the same
-for a prompt's positions 0 .. S - 1.
+for a prompt's positions 0 .. S - 1.  q after RoPE and the probabilities are
+fp32 values that enter the matrix cores as sums of two fp16 values (23 bits);
+scores, softmax and sums are fp32.
 """
 from __future__ import annotations
 

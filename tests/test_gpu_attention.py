@@ -173,3 +173,60 @@ def test_attention_queries_of_any_size(gpu, hd, size):
     _close(out, ref, "prefill")
     one = attention_decode(qkv[-1:].contiguous().to(gpu), kc, vc, cos, cos, torch.tensor([S - 1], device=gpu), nh)
     _close(one, ref[-1:], "decode")
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_scores_of_any_size(gpu, hd):
+    """Scores of up to 3e10, as far as fp16 queries and keys go: a difference of
+    two is exact to 2^-24 of itself where each is only known to some
+    thousands.  The largest wins, whether it comes first or last."""
+    nh, kvh, S = 4, 2, 150
+    cos = torch.full((S, hd), math.sqrt(0.5), device=gpu)
+    g = torch.Generator().manual_seed(hd)
+    sign = torch.where(torch.rand((1, 1, hd // 2), generator=g) < 0.5, -1.0, 1.0)
+    qkv = torch.empty((S, nh + 2 * kvh, hd))
+    qkv[:, :nh] = torch.cat((sign, -sign), -1) * 65504
+    rising = torch.arange(1, S + 1) / S
+    qkv[:, nh] = torch.cat((sign, -sign), -1)[0] * 46000 * rising.unsqueeze(1)
+    qkv[:, nh + 1] = torch.cat((sign, -sign), -1)[0] * 46000 * rising.flip(0).unsqueeze(1)
+    qkv[:, nh + kvh:] = torch.randn((S, kvh, hd), generator=g)
+    qkv = qkv.reshape(S, -1).half()
+    kc = torch.zeros((kvh, S, hd), dtype=torch.float16, device=gpu)
+    vc = kc.clone()
+    print(f"attention scores hd={hd}", flush=True)
+    out = attention_prefill(qkv.to(gpu), kc, vc, cos, cos, nh)
+    heads, c = qkv.double().view(S, -1, hd), cos.double().cpu()
+    ref = _attend64(_rope64(heads[:, :nh], c, c), kc.double().cpu(), heads[:, nh + kvh:].transpose(0, 1), 0)
+    _close(out, ref, "prefill")
+    one = attention_decode(qkv[-1:].contiguous().to(gpu), kc, vc, cos, cos, torch.tensor([S - 1], device=gpu), nh)
+    _close(one, ref[-1:], "decode")
+
+
+def test_attention_rounds_as_seldom_as_fp32(gpu):
+    """The fp32 work before the output's rounding to fp16 errs no more than
+    plain fp32 attention does: as few outputs land on another fp16 value than
+    the 64-bit result's.  Flat softmaxes, where the probabilities' own error
+    decides, and steep ones, where the scores' does."""
+    nh, kvh, hd, S = 28, 4, 128, 100
+    cos, sin = _tables(S, hd, gpu)
+    c, s = cos.cpu(), sin.cpu()
+    g = torch.Generator().manual_seed(1)
+    for std in (0.3, 1.0, 2.0):
+        other = {"prefill": [0, 0], "decode": [0, 0]}
+        for _ in range(2):
+            qkv = (torch.randn((S, (nh + 2 * kvh) * hd), generator=g) * std).half()
+            kc = torch.zeros((kvh, S, hd), dtype=torch.float16, device=gpu)
+            vc = kc.clone()
+            out = {"prefill": attention_prefill(qkv.to(gpu), kc, vc, cos, sin, nh)}
+            # the same rows one by one: the caches' rows before each are in place
+            out["decode"] = torch.cat([attention_decode(qkv[i:i + 1].to(gpu), kc, vc, cos, sin,
+                                                        torch.tensor([i], device=gpu), nh) for i in range(S)])
+            heads = qkv.view(S, -1, hd)
+            exact, plain = (_attend64(_rope64(heads[:, :nh].to(t), c.to(t), s.to(t)), kc.cpu().to(t),
+                                      heads[:, nh + kvh:].transpose(0, 1).to(t), 0).half()
+                            for t in (torch.float64, torch.float32))
+            for name, got in out.items():
+                other[name][0] += int((got.cpu() != exact).sum())
+                other[name][1] += int((plain != exact).sum())
+        print(f"attention rounding std={std}: {other} of {2 * S * nh * hd}", flush=True)
+        assert all(a <= b for a, b in other.values())
