@@ -244,9 +244,18 @@ __device__ __forceinline__ float wave_max(float v) {
     auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(i, lane)); };
     return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
 }
-// RMSNorm's factor 1 / sqrt(sum / H + eps), inv_h = 1 / H (v_rsq_f32: 1 ulp).
-__device__ __forceinline__ float norm_factor(float sum, float inv_h, float eps) {
-    return __builtin_amdgcn_rsqf(__builtin_fmaf(sum, inv_h, eps));
+// RMSNorm's factor 1 / sqrt(sum / H + eps) from eight partial sums of squares,
+// inv_h = 1 / H, rounded to fp32 once: every column of the row carries its
+// error.  The hardware's reciprocal square root, one Newton step in 64 bits
+// (some ten instructions; a correctly rounded fp32 square root and two
+// divisions are thirty, and round four times).
+__device__ __forceinline__ float norm_factor(const float (&s)[8], double inv_h, float eps) {
+    const double sum = (((double)s[0] + (double)s[1]) + ((double)s[2] + (double)s[3])) +
+                       (((double)s[4] + (double)s[5]) + ((double)s[6] + (double)s[7]));
+    const double v = __builtin_fma(sum, inv_h, (double)eps);
+    const double r = (double)__builtin_amdgcn_rsqf((float)v);
+    const double refined = __builtin_fma(0.5 * r, __builtin_fma(-v * r, r, 1.0), r);
+    return (float)(v < (double)INFINITY ? refined : r);
 }
 
 // x 2^exp = hi + lo in two fp16 values, 23 bits of it while lo stays above

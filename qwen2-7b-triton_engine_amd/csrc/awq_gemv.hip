@@ -280,7 +280,8 @@ struct QuadArgs {
     unsigned long long* fix;
     float* partials;
     const half_t* norm_w;            // kInputNorm
-    float norm_eps, norm_inv_k;
+    double norm_inv_k;
+    float norm_eps;
 };
 static_assert(offsetof(QuadArgs, out) == 64 && sizeof(QuadArgs) <= 128, "two lines");
 
@@ -477,10 +478,7 @@ __global__ __launch_bounds__(512) void awq_gemv_quad_kernel(QuadArgs a) {
         // Wave 0 also clears the places of waves that the workgroup does not have.
         if (wave == 0 ? lane == 0 || (lane >= nw && lane < 8) : lane == 0) squares[wave + lane] = lane == 0 ? s : 0.f;
         __syncthreads();
-        s = 0.f;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) s += squares[w];
-        const float r = norm_factor(s, a.norm_inv_k, a.norm_eps);
+        const float r = norm_factor(squares, a.norm_inv_k, a.norm_eps);
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             half8_t v = __builtin_bit_cast(half8_t, xv[i]);
@@ -690,7 +688,7 @@ static hipError_t gemv_quad_launch(const GemmArgs& a, const GemvConfig& cfg, uin
     q.partials = a.partials;
     q.norm_w = cfg.norm_w;
     q.norm_eps = cfg.norm_eps;
-    q.norm_inv_k = 1.0f / (float)a.K;
+    q.norm_inv_k = 1.0 / (double)a.K;
     q.total = grid.x;
     // Weight loads marked non-temporal where each workgroup streams a long
     // K range (few splits): 3584 x 37888 at split 3 measured 2.7 - 4.7 %

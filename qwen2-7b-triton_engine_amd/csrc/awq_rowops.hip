@@ -17,7 +17,7 @@ constexpr int kNormThreads = 512;
 template <int C>
 __global__ __launch_bounds__(kNormThreads) void awq_rmsnorm_kernel(const half_t* __restrict__ x,
                                                                    const half_t* __restrict__ w,
-                                                                   half_t* __restrict__ out, int H, float inv_h,
+                                                                   half_t* __restrict__ out, int H, double inv_h,
                                                                    float eps) {
     __shared__ float sums[kNormThreads / 64];
     const int pieces = H / 8;
@@ -42,10 +42,7 @@ __global__ __launch_bounds__(kNormThreads) void awq_rmsnorm_kernel(const half_t*
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = s;
     __syncthreads();
-    s = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kNormThreads / 64; ++i) s += sums[i];
-    const float r = norm_factor(s, inv_h, eps);
+    const float r = norm_factor(sums, inv_h, eps);
     half8_t* orow = reinterpret_cast<half8_t*>(out + (size_t)blockIdx.x * H);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -66,7 +63,7 @@ hipError_t launch_rmsnorm(const half_t* x, const half_t* w, half_t* out, int M, 
     if (M == 0) return hipSuccess;
     const int c = (H / 8 + kNormThreads - 1) / kNormThreads;
     auto kernel = c <= 1 ? awq_rmsnorm_kernel<1> : c <= 2 ? awq_rmsnorm_kernel<2> : awq_rmsnorm_kernel<4>;
-    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, H, 1.0f / (float)H, eps);
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, stream, x, w, out, H, 1.0 / (double)H, eps);
     return hipGetLastError();
 }
 

@@ -3,6 +3,8 @@
 Bound per element: one fp16 rounding (2^-11, or half of the smallest
 subnormal) and 1e-6 of the value for the fp32 sum of at most 16384 squares.
 """
+import math
+
 import pytest
 import torch
 
@@ -33,3 +35,21 @@ def test_rmsnorm_views_and_refusals(gpu):
     for a, b in ((x.float(), w[:528]), (x, w[:8]), (x[:, :12], w[:12]), (x.cpu(), w[:512].cpu())):
         with pytest.raises(ValueError):
             rmsnorm(a, b, 1e-5)
+
+
+@pytest.mark.parametrize("h", [256, 3584, 8192])
+def test_rmsnorm_rounds_as_seldom_as_fp32(gpu, h):
+    """The fp32 work errs no more than the same formula in plain torch fp32:
+    as few outputs land on another fp16 value than the 64-bit result's.  (Two
+    counts of about b differ by 2 sqrt(2 b) by chance: two standard deviations.)"""
+    other = [0, 0]
+    for seed in range(4):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        x = (torch.randn((4096, h), generator=g, device=gpu) * 3).half()
+        w = (1 + 0.1 * torch.randn(h, generator=g, device=gpu)).half()
+        exact, plain = ((v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + 1e-6) * w.to(v.dtype)).half()
+                        for v in (x.double(), x.float()))
+        other[0] += int((rmsnorm(x, w, 1e-6) != exact).sum())
+        other[1] += int((plain != exact).sum())
+    print(f"rmsnorm rounding h={h}: {other}", flush=True)
+    assert other[0] <= other[1] + 2 * math.sqrt(2 * other[1])
