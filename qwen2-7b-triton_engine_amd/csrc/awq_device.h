@@ -212,10 +212,15 @@ __device__ __forceinline__ void wait_batches(int n) {
 }
 
 // SiLU(x) * u in fp32 (kernels/silu_mul.py:17-39: x * sigmoid(x) * y).  The
-// hardware reciprocal (1 ulp) where a correctly rounded division takes ten
-// instructions more.
+// quotient by the hardware's reciprocal (1 ulp), corrected by its exact
+// remainder: without that a quarter more outputs land on another fp16 value
+// than the exact result's; with it every output is the correctly rounded
+// division's, at half of its instructions.  The instruction makes a subnormal
+// reciprocal 0: 2^-126 stands in for it, the quotient being far below fp16's
+// smallest value there; div_fixup sets its sign and takes infinities and NaN.
 __device__ __forceinline__ float silu_mul(float x, float u) {
-    return x * __builtin_amdgcn_rcpf(1.0f + expf(-x)) * u;
+    const float d = 1.0f + expf(-x), r = fmaxf(__builtin_amdgcn_rcpf(d), 0x1p-126f), q = x * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, x), r, q), d, x) * u;
 }
 
 // Sum over a wave, the same in every lane: DPP steps within the rows of 16

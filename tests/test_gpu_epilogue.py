@@ -104,3 +104,29 @@ def test_silu_mul_gate_up(gpu, m, i):
     two = silu_mul_forward(gu[:, :i], gu[:, i:])
     torch.cuda.synchronize()
     assert torch.equal(two, out)
+
+
+def test_silu_mul_rounds_as_seldom_as_fp32(gpu):
+    """The fp32 work errs no more than x / (1 + exp(-x)) * u with a correctly
+    rounded division: as few outputs land on another fp16 value than the
+    64-bit result's."""
+    other = [0, 0]
+    for seed in range(4):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        gu = (torch.randn((256, 2 * 18944), generator=g, device=gpu) * 4).half()
+        exact, plain = ((x / (1.0 + torch.exp(-x)) * u).half()
+                        for x, u in (gu.to(t).chunk(2, -1) for t in (torch.float64, torch.float32)))
+        other[0] += int((silu_mul_gate_up(gu) != exact).sum())
+        other[1] += int((plain != exact).sum())
+    print(f"silu_mul rounding: {other}", flush=True)
+    assert other[0] <= other[1]
+
+
+@pytest.mark.parametrize("up", [1.0, -3.0, 65504.0, 2.0**-24, 0.0, float("inf"), float("nan")])
+def test_silu_mul_every_gate(gpu, up):
+    """Every fp16 gate, infinities and NaN among them: the division's own value."""
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.float16).to(gpu)
+    got = silu_mul_gate_up(torch.cat((gate, torch.full_like(gate, up))).view(1, -1))[0]
+    x = gate.float()
+    want = (x / (1.0 + torch.exp(-x)) * up).half()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~got.isnan()], want[~want.isnan()])
