@@ -166,10 +166,8 @@ class Qwen2AwqDecoder:
         self.v_cache = torch.zeros_like(self.k_cache)
         # the HIP attention serves heads of 64 or 128 columns; torch the others
         self._hip_attention = attention_served(shape.num_heads, KV, hd, max_seq_len)
-        # the whole layer in one native call: heads and rows that the kernels
-        # serve, and this class's own projections
-        self._native_layers = (self._hip_attention and H <= MAX_H and H % 8 == 0 and
-                               type(self).linear is Qwen2AwqDecoder.linear)
+        # the whole layer in one native call: heads and rows that the kernels serve
+        self._native_layers = self._hip_attention and H <= MAX_H and H % 8 == 0
         self._graph = None
 
     # ---- linear layers: the path this build replaces -------------------------
@@ -184,7 +182,9 @@ class Qwen2AwqDecoder:
     # ---- one decoder layer over positions `pos` (device int64 [S]) -------------
     def _layer(self, li: int, h: torch.Tensor, pos: torch.Tensor, causal: bool) -> torch.Tensor:
         p = self.layers[li]
-        if self._native_layers and all(
+        # ... and the projections are this module's own: a subclass's, or one
+        # set on the class or the object at any time, is called
+        if self._native_layers and getattr(self.linear, "__func__", None) is _LINEAR and all(
                 getattr(p[k], "dtype", None) is torch.float16 for k in ("ln1", "ln2", "qkv_bias")):
             return _native.binding().qwen2_layer(h, pos, causal, p, self.k_cache[li], self.v_cache[li], self.cos,
                                                  self.sin, self.s.num_heads, self.s.rms_norm_eps)
@@ -320,3 +320,6 @@ class Qwen2AwqDecoder:
         decode_s = t2 - t1
         return {"tokens": tokens, "prefill_s": t1 - t0, "decode_s": decode_s,
                 "decode_tokens_per_s": (new_tokens - 1) / decode_s if decode_s > 0 else float("inf")}
+
+
+_LINEAR = Qwen2AwqDecoder.linear   # what qwen2_layer stands for

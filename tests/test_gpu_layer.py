@@ -70,3 +70,21 @@ def test_positions_outside_the_cache_are_refused(gpu):
         m.prefill(torch.zeros(9, dtype=torch.int64))
     m.prefill(torch.zeros(8, dtype=torch.int64))
     assert torch.equal(m.decode_logits(torch.tensor(3), torch.tensor(7)), m.decode_logits(torch.tensor(3), 7))
+
+
+def test_replaced_projections_are_called(gpu, monkeypatch):
+    """Projections set on the object or on the class after construction."""
+    m = Qwen2AwqDecoder(Qwen2Shape(num_heads=4, num_kv_heads=2, **TINY), max_seq_len=40, seed=1, device=gpu)
+    prompt, forced = torch.arange(20), torch.arange(3)
+    want, own, calls = _run(m, prompt, forced), Qwen2AwqDecoder.linear, []
+
+    def linear(self, *a, **kw):
+        calls.append(1)
+        return own(self, *a, **kw)
+
+    m.linear = linear.__get__(m)
+    assert (_run(m, prompt, forced) - want).abs().max() <= 4e-3 * want.abs().max() and len(calls) == 4 * 2 * 4
+    del m.linear
+    assert torch.equal(_run(m, prompt, forced), want) and len(calls) == 4 * 2 * 4
+    monkeypatch.setattr(Qwen2AwqDecoder, "linear", linear)
+    assert (_run(m, prompt, forced) - want).abs().max() <= 4e-3 * want.abs().max() and len(calls) == 2 * 4 * 2 * 4
