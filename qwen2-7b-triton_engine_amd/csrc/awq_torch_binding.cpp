@@ -11,7 +11,8 @@
 // reference engine makes 112 of these calls per token and never replays a
 // graph, inference/engine.py:114-139).  The checks and their messages are
 // the Python mirror's (kernels/awq_gemm.py in this package): ValueError for
-// a bad operand, RuntimeError for a failed launch.
+// a bad operand, AwqNativeError (kernels/_native.py) with the status for a
+// refused plan or a failed launch.
 //
 // gemm is the same with the bias and residual adds (awq_gemm_forward_ex's AUTO
 // path), qwen2_layer a whole decoder layer of the engine.  At M = 1 a kernel
@@ -64,8 +65,15 @@ struct PlanKeyHash {
 std::unordered_map<PlanKey, awq_w4a16_plan, PlanKeyHash> g_plans;
 std::unordered_map<int, std::vector<at::Tensor>> g_workspaces;
 
+// The Python class that check_status raises, called with (status, where); set
+// when the module is loaded and held until the process ends.
+PyObject* g_status_error = nullptr;
+
 void check_status(int st, const char* where) {
-    TORCH_CHECK(st == AWQ_OK, where, ": status ", st, ": ", awq_w4a16_error_string(st));
+    if (st == AWQ_OK) return;
+    TORCH_CHECK(g_status_error != nullptr, where, ": status ", st, ": ", awq_w4a16_error_string(st));
+    PyErr_SetObject(g_status_error, py::make_tuple(st, where).ptr());
+    throw py::error_already_set();
 }
 
 // The plan for a shape on a device (the planner sizes grids by the device's
@@ -155,7 +163,7 @@ at::Tensor run_linear(const at::Tensor& x2, const Linear& w, const at::Tensor& b
     const int st = awq_w4a16_gemm_epilogue(x2.data_ptr(), w.qweight.data_ptr<int32_t>(), w.qzeros.data_ptr<int32_t>(),
                                            w.scales.data_ptr(), data_or_null(bias), data_or_null(residual),
                                            out.data_ptr(), M, w.N, w.K, 128, ws.ptr, ws.bytes, &p, stream);
-    check_status(st, "awq_w4a16_gemm_planned");
+    check_status(st, "awq_w4a16_gemm_epilogue");
     return out;
 }
 
@@ -333,5 +341,7 @@ PYBIND11_MODULE(_awq_torch, m) {
     m.def("workspace", &workspace, "the device's workspace buffer, at least nbytes", py::arg("device_index"),
           py::arg("nbytes"));
     m.def("workspace_buffers", &workspace_buffers, "every workspace buffer of a device", py::arg("device_index"));
+    m.def("set_status_error", [](const py::object& type) { g_status_error = type.inc_ref().ptr(); },
+          "the exception class for a status of the C ABI", py::arg("type"));
     m.def("abi_version", [] { return awq_w4a16_abi_version(); });
 }

@@ -134,6 +134,7 @@ def binding():
         spec.loader.exec_module(mod)
         if mod.abi_version() != ABI_VERSION:
             raise RuntimeError(f"{path} was built against ABI {mod.abi_version()}, expected {ABI_VERSION}")
+        mod.set_status_error(AwqNativeError)
         _binding = mod
     return _binding
 

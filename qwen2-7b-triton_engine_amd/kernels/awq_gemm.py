@@ -244,10 +244,8 @@ def awq_gemm_forward_ex(x: torch.Tensor, qweight: torch.Tensor, qzeros: torch.Te
     ``residual`` fp16 ``[..., N]`` (``residual + out``, :219-227), bit-identical
     to the unfused torch adds.  ``residual`` may be ``out`` itself."""
     if path is None and plan_obj is None and out is None:
-        try:    # the AUTO plan into a new tensor: one call into the torch binding
-            return _native.binding().gemm(x, qweight, qzeros, scales, group_size, bias, residual)
-        except RuntimeError:
-            pass    # a refused plan or launch: the calls below raise it with its status
+        # the AUTO plan into a new tensor: one call into the torch binding
+        return _native.binding().gemm(x, qweight, qzeros, scales, group_size, bias, residual)
     in_shape, x_flat, qweight, qzeros, scales, K, N, dev = _prepare(x, qweight, qzeros, scales, group_size)
     M = x_flat.shape[0]
     if out is None:

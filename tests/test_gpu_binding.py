@@ -157,3 +157,15 @@ def test_binding_growth_under_capture_is_refused(gpu):
                        timeout=300)
     print(r.stdout, flush=True)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+def test_binding_raises_the_status(gpu):
+    """A shape past the kernels' 32-bit offsets: the planner's status, from both entry points."""
+    k, n = 128, 8
+    x = torch.empty((2**23 + 1, k), dtype=torch.float16, device=gpu)
+    w = (torch.zeros((k, n // 8), dtype=torch.int32, device=gpu), torch.zeros((1, n // 8), dtype=torch.int32, device=gpu),
+         torch.zeros((1, n), dtype=torch.float16, device=gpu))
+    for call in (awq_gemm_forward, awq_gemm_forward_ex):
+        with pytest.raises(_native.AwqNativeError) as e:
+            call(x, *w)
+        assert e.value.status == _native.AWQ_ERR_TOO_LARGE

@@ -659,3 +659,20 @@ def test_torch_binding_loads_and_checks_operands():
     for args, msg in cases:
         with pytest.raises(ValueError, match=msg):
             awq_gemm_forward(*args)
+
+
+def test_a_failing_binding_call_is_not_issued_again(monkeypatch):
+    """What the torch binding raises reaches the caller: out of memory, a HIP
+    error or a refused growth is no reason to take another route, which might
+    enqueue the work twice."""
+    from kernels import awq_gemm
+
+    class Failing:
+        @staticmethod
+        def gemm(*args):
+            raise RuntimeError("HIP out of memory")
+
+    monkeypatch.setattr(_native, "binding", lambda: Failing)
+    monkeypatch.setattr(awq_gemm, "_prepare", lambda *a: pytest.fail("taken again"))
+    with pytest.raises(RuntimeError, match="HIP out of memory"):
+        awq_gemm.awq_gemm_forward_ex(*(torch.zeros(1),) * 4)
