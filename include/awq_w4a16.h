@@ -350,11 +350,11 @@ int awq_fp16_rmsnorm(const void* x, const void* w, void* out, int64_t M, int64_t
  * fp16) and v stored at row *pos of the caches, softmax(q K^T / sqrt(head_dim))
  * V over positions 0 .. *pos, out fp16.  q and the probabilities enter the
  * matrix cores as sums of two fp16 values (23 bits), with fp32 sums.  qkv fp16
- * [(num_heads + 2 num_kv_heads) * head_dim]; k_cache / v_cache fp16 [num_kv_heads, max_seq,
- * head_dim]; cos / sin fp32 [max_seq, head_dim]; pos int64 [1] on the device
- * (outside 0 .. max_seq - 1 nothing is written); out fp16 [num_heads *
- * head_dim].  head_dim 64 or 128 (AWQ_ERR_PATH otherwise), num_heads a
- * multiple of num_kv_heads.  workspace: at least
+ * [(num_heads + 2 num_kv_heads) * head_dim]; k_cache / v_cache fp16
+ * [num_kv_heads, max_seq, head_dim]; cos / sin fp32 [max_seq, head_dim]; pos
+ * int64 [1] on the device (outside 0 .. max_seq - 1 the caches stay as they are
+ * and out is NaN); out fp16 [num_heads * head_dim].  head_dim 64 or 128
+ * (AWQ_ERR_PATH otherwise), num_heads a multiple of num_kv_heads.  workspace: at least
  * awq_fp16_attention_decode_workspace bytes, of any content; it holds nothing
  * between calls.  Two launches. */
 size_t awq_fp16_attention_decode_workspace(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,

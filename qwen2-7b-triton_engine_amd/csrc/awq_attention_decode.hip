@@ -264,7 +264,10 @@ __global__ __launch_bounds__(4 * HD) void awq_decode_combine_kernel(const float*
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = base[(quarter + 4 * j < ranges ? quarter + 4 * j : 0) * step + d];
     __builtin_amdgcn_sched_barrier(0);
-    if (pos < 0 || pos >= max_seq) return;
+    if (pos < 0 || pos >= max_seq) {   // the host has not seen the position: no output that could pass for one
+        if (quarter == 0) out[(size_t)head * HD + d] = (half_t)NAN;
+        return;
+    }
     const int n = (int)pos / chunk + 1;
     if (lane >= n) {
         mine = -INFINITY;

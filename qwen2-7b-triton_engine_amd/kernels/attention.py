@@ -41,7 +41,9 @@ def attention_decode(qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Te
                      sin: torch.Tensor, pos: torch.Tensor, num_heads: int) -> torch.Tensor:
     """Attention output fp16 ``[1, num_heads * head_dim]`` of the position
     ``pos`` (int64 ``[1]``, on the device); its k and v go into row ``pos`` of
-    ``k_cache`` / ``v_cache`` ``[kv_heads, max_seq, head_dim]``."""
+    ``k_cache`` / ``v_cache`` ``[kv_heads, max_seq, head_dim]``.  The host does not
+    read the position: outside the cache the caches stay as they are and the
+    output is NaN."""
     dev = qkv.device
     kvh, max_seq, hd = _check_cache(dev, k_cache, v_cache, cos, sin)
     if qkv.dtype != torch.float16 or qkv.numel() != (num_heads + 2 * kvh) * hd or not qkv.is_contiguous():

@@ -230,3 +230,16 @@ def test_attention_rounds_as_seldom_as_fp32(gpu):
                 other[name][1] += int((plain != exact).sum())
         print(f"attention rounding std={std}: {other} of {2 * S * nh * hd}", flush=True)
         assert all(a <= b for a, b in other.values())
+
+
+@pytest.mark.parametrize("max_seq", [70, 5000])      # ranges of one pass and of several
+def test_attention_decode_outside_the_cache(gpu, max_seq):
+    nh, kvh, hd = 4, 2, 64
+    cos, sin = _tables(max_seq, hd, gpu)
+    kc = torch.ones((kvh, max_seq, hd), dtype=torch.float16, device=gpu)
+    vc = kc.clone()
+    qkv = torch.full((1, (nh + 2 * kvh) * hd), 2.0, dtype=torch.float16, device=gpu)
+    for pos in (-1, max_seq, 1 << 40):
+        print(f"attention_decode max_seq={max_seq} pos={pos}", flush=True)
+        assert attention_decode(qkv, kc, vc, cos, sin, torch.tensor([pos], device=gpu), nh).isnan().all()
+        assert (kc == 1).all() and (vc == 1).all()
