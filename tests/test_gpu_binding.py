@@ -32,7 +32,7 @@ def test_binding_equals_ctypes_path(gpu, m, k, n):
     p = _native.plan_for(m, n, k)
     print(f"binding M={m} K={k} N={n} path={_native.PATH_NAMES[p.path]} v{p.variant} split={p.split_k}", flush=True)
     y = awq_gemm_forward(X, QW, QZ, S)
-    y2 = awq_gemm_forward_ex(X, QW, QZ, S, 128)
+    y2 = awq_gemm_forward_ex(X, QW, QZ, S, 128, path=_native.PATH_AUTO)   # through ctypes
     torch.cuda.synchronize()
     assert y.shape == (m, n) and y.dtype == torch.float16
     assert torch.equal(y, y2)
@@ -45,7 +45,7 @@ def test_binding_shapes_views_and_alignment(gpu):
     k, n = 3584, 4608
     x, qw, qz, s = O.make_inputs(6, k, n, seed=9)
     X, QW, QZ, S = (_t(a, gpu) for a in (x, qw, qz, s))
-    want = awq_gemm_forward_ex(X, QW, QZ, S, 128)
+    want = awq_gemm_forward_ex(X, QW, QZ, S, 128, path=_native.PATH_AUTO)   # through ctypes
     y3 = awq_gemm_forward(X.view(2, 3, k), QW, QZ, S)
     assert y3.shape == (2, 3, n) and torch.equal(y3.reshape(6, n), want)
     wide = torch.zeros((6, 2 * k), dtype=torch.float16, device=gpu)
@@ -89,7 +89,8 @@ def test_binding_workspace_registry_and_capture(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ref), f"replay {i}"
-        assert torch.equal(awq_gemm_forward(X[:4], QW, QZ, S), awq_gemm_forward_ex(X[:4], QW, QZ, S, 128))
+        assert torch.equal(awq_gemm_forward(X[:4], QW, QZ, S), awq_gemm_forward_ex(X[:4], QW, QZ, S, 128,
+                                                                                       path=_native.PATH_AUTO))
     # growing the registry under capture is refused (what earlier tests left in
     # it is unknown here, so ask for one byte more than it holds)
     have = _workspace_buffers(gpu)[-1].numel() * 4

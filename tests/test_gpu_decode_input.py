@@ -11,6 +11,7 @@ import torch
 
 from kernels import _native
 from kernels.awq_gemm import awq_gemm_decode, awq_gemm_forward_ex, decode_linear_served
+from kernels.rmsnorm import rmsnorm
 from kernels.silu_mul import silu_mul_gate_up
 from oracle import awq_oracle as O
 
@@ -48,6 +49,27 @@ def test_decode_rmsnorm(gpu, k, n):
             want = want + t.double().cpu().numpy()
             rounded = rounded + np.abs(want)
         assert (np.abs(got - want) <= 2.0**-11 * (1.01 * scale + rounded) + 2.0**-24).all()
+
+
+@pytest.mark.parametrize("k,n", [(3584, 4608), (3584, 37888), (128, 32), (1152, 4640)])
+def test_decode_rmsnorm_eps(gpu, k, n):
+    """eps as large as the row's mean square (the factor is off by 1.4 without
+    it), against 64 bits and against the norm's own kernel.  The two factors
+    differ by the order of the fp32 sum, so that about one in a thousand of the
+    row's values rounds to another fp16 value: 2^-10 of it, and all that do
+    together are less than a 32nd of sum |x w|."""
+    print(f"decode rmsnorm eps K={k} N={n}", flush=True)
+    op, w64, g = _operands(k, n, gpu)
+    x = (torch.randn((1, k), generator=g) * 1e-3).half().to(gpu)
+    nw = (1 + 0.1 * torch.randn(k, generator=g)).half().to(gpu)
+    x64 = x.double().cpu().numpy()
+    row64 = x64 / np.sqrt((x64**2).mean() + 1e-6) * nw.double().cpu().numpy()
+    y64, scale = row64 @ w64, np.abs(row64) @ np.abs(w64)
+    got = awq_gemm_decode(_native.INPUT_RMSNORM, x, *op, norm_w=nw, eps=1e-6)
+    two = awq_gemm_forward_ex(rmsnorm(x, nw, 1e-6), *op).double().cpu().numpy()
+    got = got.double().cpu().numpy()
+    assert (np.abs(got - y64) <= 2.0**-11 * (1.01 * scale + np.abs(y64)) + 2.0**-24).all()
+    assert (np.abs(got - two) <= (2.0**-10 * (scale / 32 + np.abs(y64)) + 2.0**-24)).all()
 
 
 @pytest.mark.parametrize("k,n", SHAPES)
