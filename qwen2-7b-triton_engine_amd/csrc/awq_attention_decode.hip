@@ -14,7 +14,7 @@
 // enough workgroups to load it at once, each keeps a running softmax of its
 // range for all query heads of one KV head (so K and V are read once), and a
 // second launch weights the ranges' partial sums.  Measured on Qwen2-7B's
-// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 8.4 us for
+// heads (28 of 128 over 4 KV heads, cache of 1152), graph replays: 8.7 us for
 // the two at position 1100, where two small launches take 4; 10.2 with eight
 // waves a workgroup (two per SIMD: the kernel is then bound by its own
 // instructions) and its loads behind the position's; 17 with the scores, the

@@ -6,8 +6,8 @@
 // full S x T scores in fp32 products and passed over the [heads, S, T] scores
 // in memory about eight times (matmul, scale, mask, softmax, matmul).  Here
 // the scores never leave registers.  Measured on Qwen2-7B's heads (28 of 128
-// over 4 KV heads), both launches: 30 us at S = 700, 71 us at 1777 (about 1.2
-// ms before, in some 25 launches), 264 us at 4096 -- there 0.9 PFLOP/s through
+// over 4 KV heads), both launches: 30 us at S = 700, 68 us at 1777 (about 1.2
+// ms before, in some 25 launches), 250 us at 4096 -- there 0.95 PFLOP/s through
 // the MFMA, the two parts of each operand counted; a 4-layer prefill of 1777
 // tokens 9.03 -> 4.36 ms.
 //
@@ -311,8 +311,8 @@ hipError_t launch(const PrefillAttnArgs& a, int cus, hipStream_t stream) {
     // makes twice the workgroups.  A causal grid is uneven (the last query
     // tile has all the keys) and two workgroups share a CU, so the wide tile
     // needs at least three workgroups per CU to win.  28 heads of 128 over 4
-    // KV heads, both launches, us narrow / wide: S = 1200 46 / 60, 1777 71 /
-    // 85, 4096 289 / 264.
+    // KV heads, both launches, us narrow / wide: S = 700 30 / 38, 1200 43 / 58, 1777
+    // 68 / 81, 4096 256 / 250.
     const int64_t wide = (int64_t)((a.S + 127) / 128) * a.nh, narrow = (int64_t)tiles * a.nh;
     if (wide >= 3 * cus)
         hipLaunchKernelGGL((awq_prefill_attn_kernel<HD, 2>), dim3((unsigned)wide), dim3(kThreads), 0, stream, a.qkv,

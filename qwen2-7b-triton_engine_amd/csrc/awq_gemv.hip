@@ -246,9 +246,9 @@ __global__ __launch_bounds__(512) void awq_gemv_stream_kernel(GemmArgs a, int ch
 // 7 KB from L2, and scales its own K range), kInputSiluMul takes SiLU(gate) *
 // up of its K range.  A launch in a replayed graph costs 2.1 us however small;
 // measured in graphs over 28 layers' weights, us, fused / two launches / the
-// projection alone: norm + 3584 x 4608 5.1 / 6.6 / 4.7, norm + 3584 x 37888
-// 16.7 / 17.9 / 16.0, SiLU * up + 18944 x 3584 10.5 / 12.5 / 10.2; a decoder
-// layer 46.7 / 52.5.
+// projection alone: norm + 3584 x 4608 5.1 / 6.8 / 4.8, norm + 3584 x 37888
+// 16.8 / 18.1 / 16.0, SiLU * up + 18944 x 3584 10.9 / 12.5 / 10.2; a decoder
+// layer 46.8 / 52.5.
 //
 // The way to the first load.  At 5 us a call, the time before a workgroup's
 // first weight load counts: every kernel argument line is a cold scalar load,

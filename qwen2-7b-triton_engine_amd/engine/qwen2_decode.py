@@ -15,7 +15,8 @@ and SiLU * up reads the fused gate||up output in one kernel
 (``kernels.silu_mul``); a decode step's norms and SiLU * up run in the next
 projection's prologue.  A layer is one call into the torch binding
 (``qwen2_layer``), which issues all of this; models that the kernels do not
-serve take the same steps from here.  Logits are computed for the last position only, where the
+serve, or whose ``linear`` was replaced, take the same steps from here, the norms
+and SiLU * up in launches of their own.  Logits are computed for the last position only, where the
 reference computes them for every position and keeps the last
 (``inference/engine.py:93,127``).
 
